@@ -8,6 +8,7 @@
 
 #include <type_traits>
 
+#include "qz_chain.hpp"
 #include "qz_device.hpp"
 #include "../../include/quarz_amd.h"
 
@@ -84,152 +85,6 @@ __device__ __forceinline__ Real dep_value(int comp, int cc, int j, Real t, Real 
         }
         default: return Real(0);
     }
-}
-
-// Thomas solve with factors formed beforehand, every array in LDS (Tridiag.cpp:114-125 with c', m precomputed):
-//   dp_0 = d_0 / b_0,  dp_i = (d_i - a_i dp_{i-1}) m_i,  x_{M-1} = dp_{M-1},  x_i = dp_i - c'_i x_{i+1}
-// d_i is the prepared right-hand side of FieldSolver::solve (src/FieldSolver.cpp:253-259): 0 on Dirichlet
-// rows, scale * rhs otherwise, minus fcw on the flux row.  w holds rhs on entry and dp afterwards; the
-// solution goes to x (which may be w).  Rows go in groups of four through two register sets: one group is
-// loaded while the other is computed, so the LDS latency stays off the recurrence.
-struct FwdRows { Real d0, d1, d2, d3, a0, a1, a2, a3, m0, m1, m2, m3; };
-struct BwdRows { Real p0, p1, p2, p3, c0, c1, c2, c3; };
-
-__device__ __forceinline__ void thomas_lds(const Real* a, const Real* m, const Real* cp, Real b0, Real* w, Real* x,
-                                           Real scale, bool dir0, bool dirN, bool fluxN, Real fcw, int M) {
-    const int N = M - 1;
-    Real prev = (dir0 ? Real(0) : scale * w[0]) / b0;
-    w[0] = prev;
-    auto ldf = [&](FwdRows& g, int r) {
-        g.d0 = w[r]; g.d1 = w[r + 1]; g.d2 = w[r + 2]; g.d3 = w[r + 3];
-        g.a0 = a[r]; g.a1 = a[r + 1]; g.a2 = a[r + 2]; g.a3 = a[r + 3];
-        g.m0 = m[r]; g.m1 = m[r + 1]; g.m2 = m[r + 2]; g.m3 = m[r + 3];
-    };
-    auto stepf = [&](const FwdRows& g, int r) {
-        prev = (scale * g.d0 - g.a0 * prev) * g.m0; w[r] = prev;
-        prev = (scale * g.d1 - g.a1 * prev) * g.m1; w[r + 1] = prev;
-        prev = (scale * g.d2 - g.a2 * prev) * g.m2; w[r + 2] = prev;
-        prev = (scale * g.d3 - g.a3 * prev) * g.m3; w[r + 3] = prev;
-    };
-    const int nq = (N - 1) >> 2;   // full groups of four rows in 1 .. N-1
-    int i = 1;
-    if (nq > 0) {
-        FwdRows A, B;
-        ldf(A, 1);
-        int q = 0;
-        for (; q + 2 <= nq; q += 2, i += 8) {
-            ldf(B, i + 4);
-            stepf(A, i);
-            ldf(A, (q + 2 < nq) ? i + 8 : i + 4);   // the last pass reloads rows it already holds
-            stepf(B, i + 4);
-        }
-        if (q < nq) {
-            stepf(A, i);
-            i += 4;
-        }
-    }
-    for (; i < N; ++i) {
-        prev = (scale * w[i] - a[i] * prev) * m[i];
-        w[i] = prev;
-    }
-    {
-        Real dN;
-        if (dirN) dN = Real(0);
-        else {
-            dN = scale * w[N];
-            if (fluxN) dN -= fcw;
-        }
-        prev = (dN - a[N] * prev) * m[N];
-    }
-    Real xn = prev;
-    x[N] = xn;
-    // backward: rows N-1 .. 0, groups of four from the top
-    auto ldb = [&](BwdRows& g, int r) {
-        g.p0 = w[r]; g.p1 = w[r - 1]; g.p2 = w[r - 2]; g.p3 = w[r - 3];
-        g.c0 = cp[r]; g.c1 = cp[r - 1]; g.c2 = cp[r - 2]; g.c3 = cp[r - 3];
-    };
-    auto stepb = [&](const BwdRows& g, int r) {
-        xn = g.p0 - g.c0 * xn; x[r] = xn;
-        xn = g.p1 - g.c1 * xn; x[r - 1] = xn;
-        xn = g.p2 - g.c2 * xn; x[r - 2] = xn;
-        xn = g.p3 - g.c3 * xn; x[r - 3] = xn;
-    };
-    i = N - 1;
-    const int nb = N >> 2;
-    if (nb > 0) {
-        BwdRows A, B;
-        ldb(A, i);
-        int q = 0;
-        for (; q + 2 <= nb; q += 2, i -= 8) {
-            ldb(B, i - 4);
-            stepb(A, i);
-            ldb(A, (q + 2 < nb) ? i - 8 : i - 4);
-            stepb(B, i - 4);
-        }
-        if (q < nb) {
-            stepb(A, i);
-            i -= 4;
-        }
-    }
-    for (; i >= 0; --i) {
-        xn = w[i] - cp[i] * xn;
-        x[i] = xn;
-    }
-}
-
-// Thomas factors of (L - chi) with the Dirichlet rows of FieldSolver::solve (src/FieldSolver.cpp:253-256):
-//   bw_i = b_i (Dirichlet row) or b_i - chi_i;  c'_0 = c_0 / bw_0;  m_i = 1 / (bw_i - a_i c'_{i-1});  c'_i = c_i m_i
-// Rows 0 .. N-1 from a, b, c (LDS); the last row's a_N, b_N given (the flux and Dirichlet variants of L_1
-// share every other row).  m, c' go to global memory.  Returns bw_0.
-__device__ __forceinline__ Real thomas_factor(const Real* a, const Real* b, const Real* c, const Real* chi, Real aN, Real bN,
-                              bool dir0, bool dirN, Real* __restrict__ m, Real* __restrict__ cp, int M) {
-    const int N = M - 1;
-    const Real bw0 = dir0 ? b[0] : b[0] - chi[0];
-    Real cprev = c[0] / bw0;
-    cp[0] = cprev;
-    m[0] = Real(0);
-    // rows 1 .. N-1 in groups of four through two register sets, as thomas_lds
-    struct Rows { Real w0, w1, w2, w3, a0, a1, a2, a3, c0, c1, c2, c3; };
-    auto ld = [&](Rows& g, int r) {
-        g.w0 = b[r] - chi[r]; g.w1 = b[r + 1] - chi[r + 1]; g.w2 = b[r + 2] - chi[r + 2]; g.w3 = b[r + 3] - chi[r + 3];
-        g.a0 = a[r]; g.a1 = a[r + 1]; g.a2 = a[r + 2]; g.a3 = a[r + 3];
-        g.c0 = c[r]; g.c1 = c[r + 1]; g.c2 = c[r + 2]; g.c3 = c[r + 3];
-    };
-    auto step = [&](const Rows& g, int r) {
-        Real mi;
-        mi = Real(1) / (g.w0 - g.a0 * cprev); cprev = g.c0 * mi; m[r] = mi; cp[r] = cprev;
-        mi = Real(1) / (g.w1 - g.a1 * cprev); cprev = g.c1 * mi; m[r + 1] = mi; cp[r + 1] = cprev;
-        mi = Real(1) / (g.w2 - g.a2 * cprev); cprev = g.c2 * mi; m[r + 2] = mi; cp[r + 2] = cprev;
-        mi = Real(1) / (g.w3 - g.a3 * cprev); cprev = g.c3 * mi; m[r + 3] = mi; cp[r + 3] = cprev;
-    };
-    const int nq = (N - 1) >> 2;
-    int i = 1;
-    if (nq > 0) {
-        Rows A, B;
-        ld(A, 1);
-        int q = 0;
-        for (; q + 2 <= nq; q += 2, i += 8) {
-            ld(B, i + 4);
-            step(A, i);
-            ld(A, (q + 2 < nq) ? i + 8 : i + 4);
-            step(B, i + 4);
-        }
-        if (q < nq) {
-            step(A, i);
-            i += 4;
-        }
-    }
-    for (; i < N; ++i) {
-        const Real mi = Real(1) / ((b[i] - chi[i]) - a[i] * cprev);
-        cprev = c[i] * mi;
-        m[i] = mi;
-        cp[i] = cprev;
-    }
-    const Real bwN = dirN ? bN : bN - chi[N];
-    const Real mN = Real(1) / (bwN - aN * cprev);
-    m[N] = mN;
-    cp[N] = c[N] * mN;
-    return bw0;
 }
 
 // exclusive scan of n ints in place by one wave

@@ -14,7 +14,7 @@
 //      the background and beam sources (combine_sources) (grid barrier);
 //   4. the solves: the psi / E_z / B_z systems of L0, those of L1D (m = 1) and the chi-dependent Thomas factors
 //      of the B+ operators are three jobs for three workgroups, each staging its operators in its own LDS and
-//      running its chains one lane per system (grid barrier);
+//      running its chains in one wave (qz_chain.hpp) (grid barrier);
 //   5. every workgroup forms W+ from psi and stages W+, E_z, B_z in LDS; the owned particles gather them and
 //      write their S+ contributions (grid barrier); the node sums of S+ as in 3 (grid barrier);
 //   6. the Picard iterations of B+: the systems of each operator pair are one job per workgroup, reading the
@@ -483,11 +483,12 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     }
                 }
                 __syncthreads();
-                if (w == 0 && lane < nsys) {
+                if (w < nsys / 3) {   // a DPP row per system, three per wave
                     // psi and E_z: -rhs; B_z: +rhs (FieldSolver::solve scale); L0 keeps the axis row regular
-                    const bool bz = l0 ? lane == 2 : lane >= 4;
-                    thomas_lds(a, m, cp, A.op_b[op][0], BA(3 + lane), BA(3 + lane), bz ? Real(1) : Real(-1), !l0, true,
-                               false, Real(0), M);
+                    const int sys = 3 * w + min(lane >> 4, 2);
+                    const bool bz = l0 ? sys == 2 : sys >= 4;
+                    thomas_wave(a, m, cp, A.op_b[op][0], BA(3 + sys), BA(3 + sys), bz ? Real(1) : Real(-1), !l0, true,
+                                false, Real(0), M);
                 }
                 __syncthreads();
                 // results: psi over its right-hand side in ws, E_z and B_z to their arrays
@@ -518,14 +519,14 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     }
                 }
                 __syncthreads();
-                const int nf = M1 ? 4 : 2;
-                if (w == 0 && lane < nf) {
-                    const int base = lane < 2 ? 0 : (lane == 2 ? 4 : 7);
-                    const int op = lane == 0 ? OP_L1D : lane == 1 ? OP_L1F : lane == 2 ? OP_L0 : OP_L2D;
+                if (w == 0) {
+                    const int f = min(lane >> 4, M1 ? 3 : 1);
+                    const int base = f < 2 ? 0 : (f == 2 ? 4 : 7);
+                    const int op = f == 0 ? OP_L1D : f == 1 ? OP_L1F : f == 2 ? OP_L0 : OP_L2D;
                     const Real aN = A.op_a[op][N], bN = A.op_b[op][N];
                     const bool dir0 = op != OP_L0, dirN = op != OP_L1F;
-                    g_bw0[lane] = thomas_factor(BA(base), BA(base + 1), BA(base + 2), BA(3), aN, bN, dir0, dirN,
-                                                WS(W_FAC0 + 2 * lane), WS(W_FAC0 + 2 * lane + 1), M);
+                    g_bw0[f] = thomas_factor_wave(BA(base), BA(base + 1), BA(base + 2), BA(3), aN, bN, dir0, dirN,
+                                                  WS(W_FAC0 + 2 * f), WS(W_FAC0 + 2 * f + 1), M);
                 }
                 __syncthreads();
             }
@@ -699,11 +700,12 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                         BA(7)[j] = ri;
                     }
                     __syncthreads();
-                    if (w == 0 && lane < 2) {
-                        const int f = lane == 0 ? fa : fb;
+                    if (w == 0) {
+                        const int sys = min(lane >> 4, 1);
+                        const int f = sys == 0 ? fa : fb;
                         const bool flux = f == 1;
-                        thomas_lds(BA(lane), BA(2 + 2 * lane), BA(3 + 2 * lane), g_bw0[f], BA(6 + lane), BA(6 + lane),
-                                   Real(1), f != 2, !flux, flux, flux ? fcw : Real(0), M);
+                        thomas_wave(BA(sys), BA(2 + 2 * sys), BA(3 + 2 * sys), g_bw0[f], BA(6 + sys), BA(6 + sys),
+                                    Real(1), f != 2, !flux, flux, flux ? fcw : Real(0), M);
                     }
                     __syncthreads();
                     for (int j = tid; j < M; j += mBS) {

@@ -551,29 +551,26 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
 
         // ================================================================ 5a. psi, E_z, B_z solves || chi factors
         if (w == 0) {
-            // lanes: 0 psi0, 1 ez0, 2 bz0 (L0);  m1: 3 psi1r, 4 psi1i, 5 ez1r, 6 ez1i, 7 bz1r, 8 bz1i (L1D)
-            const int njobs = M1 ? 9 : 3;
-            if (lane < njobs) {
-                const bool l0 = lane < 3;
-                const int slot = l0 ? LY::WPSI0 + lane : LY::WPSI1R + (lane - 3);
-                const Real scale = (lane == 2 || lane >= 7) ? Real(1) : Real(-1);
-                const Real b0 = l0 ? A.op_b[OP_L0][0] : A.op_b[OP_L1D][0];
-                thomas_lds(BA(l0 ? LY::L0A : LY::L1A), BA(l0 ? LY::L0M : LY::L1M), BA(l0 ? LY::L0CP : LY::L1CP), b0,
-                           BA(slot), BA(slot), scale, !l0, true, false, Real(0), M);
-            }
+            // psi0, ez0, bz0 (L0);  m1: psi1r, psi1i, ez1r, ez1i, bz1r, bz1i (L1D)
+            // (one DPP row per system, waves 0, 2 and 3)
+            const int sys = min(lane >> 4, 2);
+            thomas_wave(BA(LY::L0A), BA(LY::L0M), BA(LY::L0CP), A.op_b[OP_L0][0], BA(LY::WPSI0 + sys),
+                        BA(LY::WPSI0 + sys), sys == 2 ? Real(1) : Real(-1), false, true, false, Real(0), M);
+        } else if (M1 && (w == 2 || w == 3)) {
+            const int sys = 3 * (w - 2) + min(lane >> 4, 2);   // psi1r, psi1i, ez1r | ez1i, bz1r, bz1i
+            thomas_wave(BA(LY::L1A), BA(LY::L1M), BA(LY::L1CP), A.op_b[OP_L1D][0], BA(LY::WPSI1R + sys),
+                        BA(LY::WPSI1R + sys), sys >= 4 ? Real(1) : Real(-1), true, true, false, Real(0), M);
         } else if (w == 1) {
-            // this slice's factors of (L - chi0): lanes 0 L1D, 1 L1F, m1: 2 L0, 3 L2D
-            const int nf = M1 ? 4 : 2;
-            if (lane < nf) {
-                const Real* a = lane < 2 ? BA(LY::L1A) : lane == 2 ? BA(LY::L0A) : BA(LY::L2A);
-                const Real* b = lane < 2 ? BA(LY::L1B) : lane == 2 ? BA(LY::L0B) : BA(LY::L2B);
-                const Real* c = lane < 2 ? BA(LY::L1C) : lane == 2 ? BA(LY::L0C) : BA(LY::L2C);
-                const int op = lane == 0 ? OP_L1D : lane == 1 ? OP_L1F : lane == 2 ? OP_L0 : OP_L2D;
-                const Real aN = A.op_a[op][N], bN = A.op_b[op][N];
-                const bool dir0 = op != OP_L0, dirN = op != OP_L1F;
-                s_bw0[lane] = thomas_factor(a, b, c, BA(LY::CHI0), aN, bN, dir0, dirN, WS(W_FAC0 + 2 * lane),
-                                            WS(W_FAC0 + 2 * lane + 1), M);
-            }
+            // this slice's factors of (L - chi0), one DPP row each: L1D, L1F, m1: L0, L2D
+            const int f = min(lane >> 4, M1 ? 3 : 1);
+            const Real* a = f < 2 ? BA(LY::L1A) : f == 2 ? BA(LY::L0A) : BA(LY::L2A);
+            const Real* b = f < 2 ? BA(LY::L1B) : f == 2 ? BA(LY::L0B) : BA(LY::L2B);
+            const Real* c = f < 2 ? BA(LY::L1C) : f == 2 ? BA(LY::L0C) : BA(LY::L2C);
+            const int op = f == 0 ? OP_L1D : f == 1 ? OP_L1F : f == 2 ? OP_L0 : OP_L2D;
+            const Real aN = A.op_a[op][N], bN = A.op_b[op][N];
+            const bool dir0 = op != OP_L0, dirN = op != OP_L1F;
+            s_bw0[f] = thomas_factor_wave(a, b, c, BA(LY::CHI0), aN, bN, dir0, dirN, WS(W_FAC0 + 2 * f),
+                                          WS(W_FAC0 + 2 * f + 1), M);
         }
         __syncthreads();
         QZ_PHASE(6);
@@ -806,16 +803,15 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
                 }
                 __syncthreads();
                 QZ_PHASE(12);
-                // lanes: 0 B_r1 (L1D), 1 B_i1 (L1F, flux wall J_z(R)); m1: 2 B_r0, 3 B_i0 (L0), 4 B_r2, 5 B_i2 (L2D)
-                if (w == 0) {
-                    const int nj = M1 ? 6 : 2;
-                    if (lane < nj) {
-                        const int fidx = lane < 2 ? lane : (lane < 4 ? 2 : 3);   // factor set: L1D, L1F, L0, L2D
-                        const Real* a = BA(fidx == 0 ? LY::PA_L1D : fidx == 1 ? LY::PA_L1F : fidx == 2 ? LY::PA_L0 : LY::PA_L2D);
-                        const bool flux = fidx == 1;
-                        thomas_lds(a, BA(LY::PF + 2 * fidx), BA(LY::PF + 2 * fidx + 1), s_bw0[fidx], BA(LY::PRB + lane),
-                                   BA(LY::PBP + lane), Real(1), fidx != 2, !flux, flux, flux ? fcw : Real(0), M);
-                    }
+                // systems: 0 B_r1 (L1D), 1 B_i1 (L1F, flux wall J_z(R)); m1: 2 B_r0, 3 B_i0 (L0), 4 B_r2, 5 B_i2 (L2D),
+                // two (m1: three) DPP rows of wave 0 (and wave 1)
+                if (w < (M1 ? 2 : 1)) {
+                    const int sys = M1 ? 3 * w + min(lane >> 4, 2) : min(lane >> 4, 1);
+                    const int fidx = sys < 2 ? sys : (sys < 4 ? 2 : 3);   // factor set: L1D, L1F, L0, L2D
+                    const Real* a = BA(fidx == 0 ? LY::PA_L1D : fidx == 1 ? LY::PA_L1F : fidx == 2 ? LY::PA_L0 : LY::PA_L2D);
+                    const bool flux = fidx == 1;
+                    thomas_wave(a, BA(LY::PF + 2 * fidx), BA(LY::PF + 2 * fidx + 1), s_bw0[fidx], BA(LY::PRB + sys),
+                                BA(LY::PBP + sys), Real(1), fidx != 2, !flux, flux, flux ? fcw : Real(0), M);
                 }
             }
         }
