@@ -8,11 +8,11 @@
 //   - laser_factor_kernel and laser_march_kernel (Laser::advance_slice, :317-419): the Crank-Nicolson step in t of
 //     every slice, marched from the head of the box.  Slice k needs X = a^(n+1) - a^n of slices k-1 and k-2, so
 //     the march is serial in xi and runs in one workgroup: per slice the workgroup forms the right-hand sides of
-//     all nodes in LDS, one lane runs the right-hand side's Thomas recurrence and the back substitution (serial
+//     all nodes in LDS, one wave runs the right-hand side's Thomas recurrence and the back substitution (serial
 //     chains, as in the reference), and the workgroup forms the carry and a^(n+1).  The pivots and c' of the
 //     recurrence depend only on the slice's susceptibility, so the factor kernel forms them beforehand for all
 //     slices at once, one thread per slice, and the march's serial chain holds one complex division per node
-//     instead of two.  The carry and the right-hand sides never leave LDS.
+//     instead of two.  The carry stays in registers and the right-hand sides in LDS.
 //
 // The arithmetic of each node follows the reference's expressions in the same order (no contraction), so the
 // result equals the serial CPU restatement bit for bit.  Scope: laser.l = 0 (no vortex), no ionization losses,
@@ -43,10 +43,9 @@ __device__ __forceinline__ Cx cdiv(Cx a, Cx b) {
 constexpr int kPondThreads = 256;
 constexpr int kFactorThreads = 64;
 constexpr int kMarchThreads = 512;
-// LDS doubles per node of the march: c' (2), pivot (2), rhs / d' / X (2), the carry (4), -a_j (1)
-constexpr int kMarchLdsPerNode = 11;
 constexpr long kMaxLds = 160 * 1024;
-constexpr int kMaxNodes = 1861;   // 11 doubles per node in 160 KB
+constexpr int kMaxNodes = 1861;   // 11 doubles per node in 160 KB (MarchLds)
+static_assert(kMaxNodes <= 4 * kMarchThreads, "a thread of the march owns at most four nodes");
 
 // the diagonal's constant part, cd 2/(dt dxi) - 4 i k0 / dt (src/Laser.cpp:352-361)
 __device__ __forceinline__ Cx march_alpha(double dxi, double dt, double k0, int scheme) {
@@ -105,116 +104,325 @@ __device__ __forceinline__ void factor_slice(int k, const double* __restrict__ c
     }
 }
 
-// One workgroup marches the K slices of one box.  Every barrier is reached by all threads in every slice.
+// the other lane's value within each pair of lanes (0 with 1): the real and imaginary parts of one complex number
+__device__ __forceinline__ double pair_swap(double x) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0xB1, 0xF, 0xF, true);   // quad_perm [1, 0, 3, 2]
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), 0xB1, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+// `src` of the pair of lanes before (after) this one among the 16 of a DPP row; the first (last) pair keeps `edge`
+__device__ __forceinline__ double pair_prev(double edge, double src) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(src), 0x112, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(src), 0x112, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double pair_next(double edge, double src) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(edge), __double2loint(src), 0x102, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(edge), __double2hiint(src), 0x102, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+// the last pair's value to the first (the first's to the last), by a rotation of the DPP row
+__device__ __forceinline__ double pair_ror(double x) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0x122, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), 0x122, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double pair_rol(double x) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0x12E, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), 0x12E, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+constexpr int kMarchR = 8;                  // nodes per pair of lanes in the chain
+constexpr int kMarchBlock = 8 * kMarchR;
+__device__ __forceinline__ double sign_flip(double x, int signbit) {
+    return __hiloint2double(__double2hiint(x) ^ signbit, __double2loint(x));
+}
+__device__ __forceinline__ bool same_bits(double a, double b) {
+    return __double_as_longlong(a) == __double_as_longlong(b);
+}
+
+// LDS of a march, in doubles: per node of 0 .. N-1 the pivot (re, im), its |m|^2 and 1 / |m|^2, c' and -a_j; per node
+// of 0 .. N the right-hand side (then d') and X, real and imaginary parts in arrays of their own; a flag
+struct MarchLds {
+    int Ne, Me, mm, dy, cp, low, dre, xre, flag, total;
+    __host__ __device__ explicit MarchLds(int M) {
+        Ne = M & ~1;   // N = M - 1 rounded up to even
+        Me = (M + 1) & ~1;
+        mm = 0;
+        dy = mm + 2 * Ne;
+        cp = dy + 2 * Ne;
+        low = cp + 2 * Ne;
+        dre = low + Ne;
+        xre = dre + 2 * Me;
+        flag = xre + 2 * Me;
+        total = flag + 1;
+    }
+};
+
+// One workgroup marches the K slices of one box; thread tid owns nodes tid + u kMarchThreads, u < NPT.  The
+// serial chain of a slice (d'_j = (rhs_j + a_j d'_{j-1}) / m_j, then the back substitution) bounds the march: it runs
+// in one wave, which issues an instruction every four cycles at best, so its instruction count is its time.  A pair
+// of lanes forms a node's real and imaginary parts.  As in qz_chain.hpp, 8 pairs hold 8 consecutive nodes each in
+// registers and repeat their nodes on the value that the pair before them had after the last step: after 8 steps it has
+// passed through 64 nodes, which cost one set of LDS accesses (an LDS read costs the wave 9 to 14 cycles, a write 13 to
+// 27; one pair walking the nodes through LDS took 186 cycles per node).  A quotient n / |m|^2 in the chain is n y corrected once by its exact
+// residual, y = 1 / |m|^2 formed beforehand: three dependent operations against about twelve of a division.  The
+// correction gives the correctly rounded quotient but for operands at the ends of the exponent range, so while the
+// back substitution runs the other waves divide every node's numerator again with the IEEE division and compare the
+// bits; a slice with any difference has its chain run again with that division.  The next slice's rows and envelope
+// are loaded into registers while the chain runs, and the carry stays in its owner's registers.
+// Measured on 401 slices x 321 nodes (bdf2): 6.8 ms a step, 41e3 cycles per slice, where one lane dividing in the
+// chain took 30.8 ms.
+// Every barrier is reached by all threads in every slice.
+template <int NPT>
 __device__ __forceinline__ void march_box(const double* __restrict__ a, const double* __restrict__ chi,
                                           double* __restrict__ an, const double* __restrict__ la,
                                           const double* __restrict__ lb, const double* __restrict__ lc,
                                           const double* __restrict__ fac, int K, int M, double dxi, double dt,
                                           double k0, int scheme) {
     extern __shared__ double lds[];
-    Cx* cpl = reinterpret_cast<Cx*>(lds);   // c' of the slice
-    Cx* ml = cpl + M;                       // pivots m of the slice
-    Cx* rhs = ml + M;                       // rhs, then d', then X
-    Cx* car0 = rhs + M;                     // X of the previous slice
-    Cx* car1 = car0 + M;                    // G of the previous slice (trapezoid) or X two slices back
-    double* low = reinterpret_cast<double*>(car1 + M);   // -a_j (0 at j = 0)
+    const MarchLds P(M);
+    double2* const ml = reinterpret_cast<double2*>(lds + P.mm);
+    double2* const dyl = reinterpret_cast<double2*>(lds + P.dy);   // |m|^2, 1 / |m|^2
+    double2* const cpl = reinterpret_cast<double2*>(lds + P.cp);
+    double* const low = lds + P.low;
+    double* const dre = lds + P.dre;
+    double* const dim = dre + P.Me;
+    double* const xre = lds + P.xre;
+    double* const xim = xre + P.Me;
+    int* const bad = reinterpret_cast<int*>(lds + P.flag);
     const int tid = threadIdx.x, N = M - 1;
     // src/Laser.cpp:352-361
     const double c1 = scheme == 0 ? 4.0 : (scheme == 1 ? 4.0 : 2.0);
     const double c2 = scheme == 1 ? -1.0 : 0.0;
     const double s0 = 2.0 / (dt * dxi);
     const double s2 = 4.0 / dt;
-    for (int j = tid; j < M; j += kMarchThreads) {
-        car0[j] = Cx{0.0, 0.0};
-        car1[j] = Cx{0.0, 0.0};
-        const double aj = j > 0 ? la[j] : 0.0;
-        low[j] = -aj;
-    }
-    __syncthreads();
-    for (int k = 0; k < K; ++k) {
+    // owned nodes: operator rows, carry (X of the previous slice; G of it (trapezoid) or X two slices back), and the
+    // coming slice's envelope around the node, rows and susceptibility
+    double aj[NPT], bj[NPT], cj[NPT], hc[NPT];
+    Cx car0[NPT], car1[NPT], am[NPT], a0[NPT], ap[NPT], fm[NPT], fc[NPT];
+    auto load = [&](int k) {
         const double* ak = a + static_cast<long>(k) * M * 2;
-        const double* ch = chi ? chi + static_cast<long>(k) * M : nullptr;
-        double* ank = an + static_cast<long>(k) * M * 2;
-        auto A = [&](int j) { return Cx{ak[2 * j], ak[2 * j + 1]}; };
-        // the right-hand side of node j: hist + 2 H a^n (src/Laser.cpp:371-384); the slice's pivots and c' into LDS
         const double* fk = fac + static_cast<long>(k) * N * 4;
-        for (int j = tid; j < N; j += kMarchThreads) {
-            const double* f = fk + static_cast<long>(j) * 4;
-            ml[j] = Cx{f[0], f[1]};
-            cpl[j] = Cx{f[2], f[3]};
-            const double aj = j > 0 ? la[j] : 0.0, bj = lb[j], cj = lc[j];
-            const Cx hd{bj - (ch ? ch[j] : 0.0), 0.0};
-            Cx Ha = cmul(hd, A(j));
-            if (j > 0) Ha = cadd(Ha, cscale(aj, A(j - 1)));
-            Ha = cadd(Ha, cscale(cj, A(j + 1)));
-            const Cx xp = car0[j], gp = car1[j];
+#pragma unroll
+        for (int u = 0; u < NPT; ++u) {
+            // nodes past the wall repeat it: every load is issued before the first is waited for
+            const int j = min(tid + u * kMarchThreads, N), jl = max(j - 1, 0), jr = min(j + 1, N), jn = min(j, N - 1);
+            a0[u] = Cx{ak[2 * j], ak[2 * j + 1]};
+            am[u] = Cx{ak[2 * jl], ak[2 * jl + 1]};
+            ap[u] = Cx{ak[2 * jr], ak[2 * jr + 1]};
+            const double* f = fk + static_cast<long>(jn) * 4;
+            fm[u] = Cx{f[0], f[1]};
+            fc[u] = Cx{f[2], f[3]};
+            hc[u] = chi ? chi[static_cast<long>(k) * M + j] : 0.0;
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < NPT; ++u) {
+        const int j = tid + u * kMarchThreads;
+        aj[u] = bj[u] = cj[u] = 0.0;
+        car0[u] = car1[u] = Cx{0.0, 0.0};
+        if (j < N) {
+            aj[u] = j > 0 ? la[j] : 0.0;
+            bj[u] = lb[j];
+            cj[u] = lc[j];
+            low[j] = -aj[u];
+        }
+    }
+    if (tid == 0) *bad = 0;
+    load(0);
+    for (int k = 0; k < K; ++k) {
+        double* ank = an + static_cast<long>(k) * M * 2;
+        Cx r[NPT], A0[NPT], Am[NPT], Ap[NPT];   // this slice's right-hand side and envelope
+        double hdr[NPT];
+        // the right-hand side: hist + 2 H a^n (src/Laser.cpp:371-384); the slice's pivots and c' into LDS
+#pragma unroll
+        for (int u = 0; u < NPT; ++u) {
+            const int j = tid + u * kMarchThreads;
+            A0[u] = a0[u]; Am[u] = am[u]; Ap[u] = ap[u];
+            hdr[u] = bj[u] - hc[u];
+            r[u] = Cx{0.0, 0.0};
+            if (j >= N) continue;
+            const Cx m = fm[u];
+            const double d = m.re * m.re + m.im * m.im;
+            ml[j] = make_double2(m.re, m.im);
+            dyl[j] = make_double2(d, 1.0 / d);
+            cpl[j] = make_double2(fc[u].re, fc[u].im);
+            const Cx hd{hdr[u], 0.0};
+            Cx Ha = cmul(hd, A0[u]);
+            if (j > 0) Ha = cadd(Ha, cscale(aj[u], Am[u]));
+            Ha = cadd(Ha, cscale(cj[u], Ap[u]));
+            const Cx xp = car0[u], gp = car1[u];
             const Cx hist = scheme == 0 ? cadd(cscale(c1 * s0, xp), cscale(s2, gp))
                                         : cadd(cscale(c1 * s0, xp), cscale(c2 * s0, gp));
-            rhs[j] = cadd(hist, cscale(2.0, Ha));
+            r[u] = cadd(hist, cscale(2.0, Ha));
+            dre[j] = r[u].re;
+            dim[j] = r[u].im;
         }
         __syncthreads();
-        // d'_j = (rhs_j + a_j d'_{j-1}) / m_j with the slice's pivots, then back substitution (src/Laser.cpp:385-399),
-        // X_N = 0.  Node j +- 1's operands are read from LDS before node j is formed, so the chain does not wait
-        // for LDS.
-        if (tid == 0) {
-            Cx dprev{0.0, 0.0};
-            Cx m_n = ml[0], r_n = rhs[0];
-            double lo_n = low[0];
-            for (int j = 0; j < N; ++j) {
-                const Cx m = m_n, r = r_n;
-                const double lo = lo_n;
-                if (j + 1 < N) {
-                    m_n = ml[j + 1];
-                    r_n = rhs[j + 1];
-                    lo_n = low[j + 1];
+        if (k + 1 < K) load(k + 1);
+        const int p = tid & 1, g = (tid >> 1) & 7;
+        const int neg_im = p ? static_cast<int>(0x80000000u) : 0, neg_re = p ? 0 : static_cast<int>(0x80000000u);
+        if (tid < 16) {   // d' from the axis outwards
+            double* const D = p ? dim : dre;
+            double carry = 0.0;
+            for (int b0 = 0; b0 < N; b0 += kMarchBlock) {
+                const int i0 = b0 + g * kMarchR, last = P.Ne - 2;
+                double mre[kMarchR], mim[kMarchR], dd[kMarchR], yy[kMarchR], lo[kMarchR], rr[kMarchR], dv[kMarchR];
+#pragma unroll
+                for (int t = 0; t < kMarchR; t += 2) {
+                    const int i = min(i0 + t, last);
+                    const double2 l2 = *reinterpret_cast<const double2*>(low + i);
+                    const double2 r2 = *reinterpret_cast<const double2*>(D + i);
+                    lo[t] = l2.x; lo[t + 1] = l2.y;
+                    rr[t] = r2.x; rr[t + 1] = r2.y;
+#pragma unroll
+                    for (int v = 0; v < 2; ++v) {
+                        const double2 m2 = ml[i + v], d2 = dyl[i + v];
+                        mre[t + v] = m2.x;
+                        mim[t + v] = sign_flip(m2.y, neg_im);
+                        dd[t + v] = d2.x;
+                        yy[t + v] = d2.y;
+                    }
                 }
-                const Cx dpj = cdiv(csub(r, cscale(lo, dprev)), m);
-                rhs[j] = dpj;
-                dprev = dpj;
-            }
-            rhs[N] = Cx{0.0, 0.0};
-            Cx xn{0.0, 0.0};
-            Cx c_n = cpl[N - 1], d_n = rhs[N - 1];
-            for (int j = N - 1; j >= 0; --j) {
-                const Cx cp = c_n, dp = d_n;
-                if (j > 0) {
-                    c_n = cpl[j - 1];
-                    d_n = rhs[j - 1];
+                if (b0 + kMarchBlock > N) {   // no nodes from N on: d' = 0
+#pragma unroll
+                    for (int t = 0; t < kMarchR; ++t)
+                        if (i0 + t >= N) {
+                            lo[t] = rr[t] = mim[t] = 0.0;
+                            mre[t] = dd[t] = yy[t] = 1.0;
+                        }
                 }
-                const Cx x = csub(dp, cmul(cp, xn));
-                rhs[j] = x;
-                xn = x;
+                const int steps = min(8, (N - b0 + kMarchR - 1) / kMarchR);
+                double q = carry;
+                dv[kMarchR - 1] = 0.0;
+#pragma unroll 1
+                for (int st = 0; st < steps; ++st) {
+                    q = pair_prev(q, dv[kMarchR - 1]);
+                    double dp = q;
+#pragma unroll
+                    for (int t = 0; t < kMarchR; ++t) {
+                        const double sv = rr[t] - lo[t] * dp;
+                        const double num = sv * mre[t] + pair_swap(sv) * mim[t];
+                        const double q0 = num * yy[t];
+                        dp = __builtin_fma(__builtin_fma(-dd[t], q0, num), yy[t], q0);
+                        dv[t] = dp;
+                    }
+                }
+#pragma unroll
+                for (int t = 0; t < kMarchR; t += 2)
+                    if (i0 + t < N) *reinterpret_cast<double2*>(D + i0 + t) = make_double2(dv[t], dv[t + 1]);
+                carry = pair_ror(dv[kMarchR - 1]);
             }
         }
         __syncthreads();
-        // the carry for the next slice and a^(n+1) = a^n + X (src/Laser.cpp:400-418)
-        for (int j = tid; j <= N; j += kMarchThreads) {
-            const Cx X = rhs[j];
-            const Cx an_j = A(j);
+        if (tid < 16) {   // back substitution (src/Laser.cpp:394-399), X_N = 0
+            const double* const D = p ? dim : dre;
+            double* const X = p ? xim : xre;
+            double carry = 0.0;
+            for (int b0 = (N - 1) / kMarchBlock * kMarchBlock; b0 >= 0; b0 -= kMarchBlock) {
+                const int i0 = b0 + g * kMarchR, last = P.Ne - 2;
+                double cre[kMarchR], cim[kMarchR], dv[kMarchR], xv[kMarchR];
+#pragma unroll
+                for (int t = 0; t < kMarchR; t += 2) {
+                    const int i = min(i0 + t, last);
+                    const double2 d2 = *reinterpret_cast<const double2*>(D + i);
+                    dv[t] = d2.x; dv[t + 1] = d2.y;
+#pragma unroll
+                    for (int v = 0; v < 2; ++v) {
+                        const double2 c2 = cpl[i + v];
+                        cre[t + v] = c2.x;
+                        cim[t + v] = sign_flip(c2.y, neg_re);
+                    }
+                }
+                if (b0 + kMarchBlock > N) {   // X = 0 from N on
+#pragma unroll
+                    for (int t = 0; t < kMarchR; ++t)
+                        if (i0 + t >= N) cre[t] = cim[t] = dv[t] = 0.0;
+                }
+                const int steps = min(8, (N - b0 + kMarchR - 1) / kMarchR);
+                double q = carry;
+                xv[0] = 0.0;
+#pragma unroll 1
+                for (int st = 0; st < steps; ++st) {
+                    q = pair_next(q, xv[0]);
+                    double x = q;
+#pragma unroll
+                    for (int t = kMarchR - 1; t >= 0; --t) {
+                        x = dv[t] - (cre[t] * x + cim[t] * pair_swap(x));
+                        xv[t] = x;
+                    }
+                }
+#pragma unroll
+                for (int t = 0; t < kMarchR; t += 2)
+                    if (i0 + t < M) *reinterpret_cast<double2*>(X + i0 + t) = make_double2(xv[t], xv[t + 1]);
+                carry = pair_rol(xv[0]);
+            }
+            if (g == 0) X[N] = 0.0;
+        }
+        // every d' against the IEEE division
+        auto quotient = [&](Cx rr, double lo, Cx dprev, Cx m) { return cdiv(csub(rr, cscale(lo, dprev)), m); };
+#pragma unroll
+        for (int u = 0; u < NPT; ++u) {
+            const int j = tid + u * kMarchThreads;
+            if (j >= N) continue;
+            const Cx dprev = j > 0 ? Cx{dre[j - 1], dim[j - 1]} : Cx{0.0, 0.0};
+            const Cx q = quotient(r[u], -aj[u], dprev, Cx{ml[j].x, ml[j].y});
+            if (!same_bits(q.re, dre[j]) || !same_bits(q.im, dim[j])) *bad = 1;
+        }
+        __syncthreads();
+        if (*bad) {   // uniform: the slice's chain again, divided (operands at the ends of the exponent range)
+#pragma unroll
+            for (int u = 0; u < NPT; ++u) {
+                const int j = tid + u * kMarchThreads;
+                if (j < N) {
+                    dre[j] = r[u].re;
+                    dim[j] = r[u].im;
+                }
+            }
+            __syncthreads();
+            if (tid == 0) {
+                *bad = 0;
+                Cx dp{0.0, 0.0}, x{0.0, 0.0};
+                for (int j = 0; j < N; ++j) {
+                    dp = quotient(Cx{dre[j], dim[j]}, low[j], dp, Cx{ml[j].x, ml[j].y});
+                    dre[j] = dp.re;
+                    dim[j] = dp.im;
+                }
+                for (int j = N - 1; j >= 0; --j) {
+                    x = csub(Cx{dre[j], dim[j]}, cmul(Cx{cpl[j].x, cpl[j].y}, x));
+                    xre[j] = x.re;
+                    xim[j] = x.im;
+                }
+            }
+            __syncthreads();
+        }
+        // the carry for the next slice and a^(n+1) = a^n + X (src/Laser.cpp:400-418).  The next slice's first phase
+        // writes the pivots and right-hand sides, which nothing reads any more; X is written after its barrier.
+#pragma unroll
+        for (int u = 0; u < NPT; ++u) {
+            const int j = tid + u * kMarchThreads;
+            if (j > N) continue;
+            const Cx X{xre[j], xim[j]};
             if (scheme != 0) {
-                car1[j] = car0[j];
-                car0[j] = X;
+                car1[u] = car0[u];
+                car0[u] = X;
             } else {
                 Cx G{0.0, 0.0};
                 if (j < N) {
-                    auto Y = [&](int jj) {
-                        const Cx x = rhs[jj];
-                        return Cx{x.re + 2.0 * ak[2 * jj], x.im + 2.0 * ak[2 * jj + 1]};
-                    };
-                    const double aj = j > 0 ? la[j] : 0.0, bj = lb[j], cj = lc[j];
-                    const Cx hd{bj - (ch ? ch[j] : 0.0), 0.0};
-                    Cx HY = cmul(hd, Y(j));
-                    if (j > 0) HY = cadd(HY, cscale(aj, Y(j - 1)));
-                    HY = cadd(HY, cscale(cj, Y(j + 1)));
+                    auto Y = [&](Cx av, int jj) { return Cx{xre[jj] + 2.0 * av.re, xim[jj] + 2.0 * av.im}; };
+                    const Cx hd{hdr[u], 0.0};
+                    Cx HY = cmul(hd, Y(A0[u], j));
+                    if (j > 0) HY = cadd(HY, cscale(aj[u], Y(Am[u], j - 1)));
+                    HY = cadd(HY, cscale(cj[u], Y(Ap[u], j + 1)));
                     G = cadd(cmul(Cx{0.0, k0}, X), cscale(0.25 * dt, HY));
                 }
-                car0[j] = X;
-                car1[j] = G;
+                car0[u] = X;
+                car1[u] = G;
             }
-            ank[2 * j] = X.re + an_j.re;
-            ank[2 * j + 1] = X.im + an_j.im;
+            ank[2 * j] = X.re + A0[u].re;
+            ank[2 * j + 1] = X.im + A0[u].im;
         }
-        __syncthreads();
     }
 }
 
@@ -251,10 +459,16 @@ template <bool kBatch>
 __global__ __launch_bounds__(kMarchThreads) void laser_march_kernel(LaserBox one, const LaserBox* __restrict__ many) {
     const LaserBox B = kBatch ? many[blockIdx.x] : one;
     if (!B.active) return;   // the whole workgroup, before any barrier
-    march_box(B.a, B.chi, B.an, B.la, B.lb, B.lc, B.fac, B.K, B.M, B.dxi, B.dt, B.k0, B.scheme);
+    // nodes per thread: a box of at most 512 nodes keeps one node's rows in registers
+    if (B.M <= kMarchThreads)
+        march_box<1>(B.a, B.chi, B.an, B.la, B.lb, B.lc, B.fac, B.K, B.M, B.dxi, B.dt, B.k0, B.scheme);
+    else if (B.M <= 2 * kMarchThreads)
+        march_box<2>(B.a, B.chi, B.an, B.la, B.lb, B.lc, B.fac, B.K, B.M, B.dxi, B.dt, B.k0, B.scheme);
+    else
+        march_box<4>(B.a, B.chi, B.an, B.la, B.lb, B.lc, B.fac, B.K, B.M, B.dxi, B.dt, B.k0, B.scheme);
 }
 
-long march_lds(int M) { return static_cast<long>(kMarchLdsPerNode) * M * static_cast<long>(sizeof(double)); }
+long march_lds(int M) { return static_cast<long>(MarchLds(M).total) * static_cast<long>(sizeof(double)); }
 
 // glibc exp / cos / sin called through pointers, so that no compiler folds or replaces them: the pulse is
 // formed from the C library's values at run time, as the CPU restatement forms it
