@@ -44,6 +44,14 @@ __device__ __forceinline__ Real dpp_rol(Real src) {
     return __hiloint2double(hi, lo);
 }
 
+// 1 / d by the hardware's estimate (a relative error of at most 2^-24) and two Newton steps: the correctly rounded value
+// but for about one operand in 2^42, and at the ends of the exponent range
+__device__ __forceinline__ Real chain_recip(Real d) {
+    const Real y0 = __builtin_amdgcn_rcp(d);
+    const Real y1 = __builtin_fma(__builtin_fma(-d, y0, Real(1)), y0, y0);
+    return __builtin_fma(__builtin_fma(-d, y1, Real(1)), y1, y1);
+}
+
 // rows i .. i + R - 1 (i even) of an LDS array of M values padded to an even count and aligned to 16 bytes; rows from
 // M on repeat the array's last pair
 template <int R> __device__ __forceinline__ void chain_load(const Real* p, int i, int M, Real (&v)[R]) {
@@ -155,10 +163,8 @@ __device__ __forceinline__ void thomas_wave(const Real* a, const Real* m, const 
 //   bw_i = b_i (Dirichlet row) or b_i - chi_i;  c'_0 = c_0 / bw_0;  m_i = 1 / (bw_i - a_i c'_{i-1});  c'_i = c_i m_i
 // Rows 0 .. N-1 from a, b, c (LDS); the last row's a_N, b_N given (the flux and Dirichlet variants of L_1
 // share every other row).  m, c' go to global memory.  Returns bw_0.  Called as thomas_wave.
-// The reciprocal in the chain is the hardware's estimate (a relative error of at most 2^-24) with two Newton steps,
-// whose result differs from the correctly rounded one about once in 2^42 operands, and at the ends of the exponent
-// range; after its steps a block is divided once more with the IEEE division, all its rows at once, and one with
-// any difference is run again with that division in the chain.
+// The reciprocal in the chain is chain_recip; after its steps a block is divided once more with the IEEE division, all
+// its rows at once, and one with any difference is run again with that division in the chain.
 // Measured: 513 rows 16.8 us, 257 rows 9.1 us, where one lane per system dividing in the chain took 48 and 23 us.
 __device__ __forceinline__ Real thomas_factor_wave(const Real* a, const Real* b, const Real* c, const Real* chi, Real aN,
                                                    Real bN, bool dir0, bool dirN, Real* __restrict__ m,
@@ -204,11 +210,7 @@ __device__ __forceinline__ Real thomas_factor_wave(const Real* a, const Real* b,
                 pv[r] = p;
             }
         };
-        auto newton = [](Real d) {
-            const Real y0 = __builtin_amdgcn_rcp(d);
-            const Real y1 = __builtin_fma(__builtin_fma(-d, y0, Real(1)), y0, y0);
-            return __builtin_fma(__builtin_fma(-d, y1, Real(1)), y1, y1);
-        };
+        auto newton = [](Real d) { return chain_recip(d); };
         auto divide = [](Real d) { return Real(1) / d; };
         Real q = carry;
         pv[R - 1] = Real(0);

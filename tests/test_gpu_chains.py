@@ -33,6 +33,43 @@ def test_rows(qa, oracle, decks, N, modes, groups):
         assert a.shape == b.shape and np.array_equal(a, b), (w, np.argwhere(a != b)[:3])
 
 
+@pytest.mark.parametrize("layout", ["rows", "rows padded", "element-major"])
+@pytest.mark.parametrize("M,batch", [(1, 5), (2, 1), (7, 3), (8, 4), (9, 5), (127, 6), (128, 4), (129, 9), (257, 2), (1025, 5),
+                                     (33, 4097)])
+def test_thomas_layouts(qa, oracle, M, batch, layout):
+    """thomas_batched and the strided entry point: the last rows' pairs and blocks, batches that leave a wave's DPP rows
+    empty, both kernels of element-major systems, and systems whose pivots leave the reciprocal's range."""
+    import torch
+    rng = np.random.default_rng(M * 7 + batch)
+    a, c, d = (rng.uniform(-1, 1, (batch, M)) for _ in range(3))
+    b = 2.5 + rng.uniform(-1, 1, (batch, M))
+    for s, e in ((0, 1e-310), (1, 1e305), (2, 1e-305)):
+        if s < batch:
+            a[s], b[s], c[s] = a[s] * e, b[s] * e, c[s] * e
+    a[:, 0], c[:, -1] = np.inf, np.nan   # not used
+    with np.errstate(all="ignore"):
+        n = min(batch, 9)
+        ref = [oracle.thomas(np.r_[0.0, a[s, 1:]], b[s].copy(), np.r_[c[s, :-1], 0.0], d[s].copy()) for s in range(n)]
+    width = M + 3 if layout == "rows padded" else M
+    host = [np.pad(v, ((0, 0), (0, width - M))) for v in (a, b, c, d)]
+    if layout == "element-major":
+        host = [np.ascontiguousarray(v.T) for v in host]
+    dev = [torch.from_numpy(v).cuda() for v in host]
+    x = torch.zeros_like(dev[3])
+    work = torch.empty(max(1, qa.lib().qz_tridiag_workspace_doubles(M, batch)), dtype=torch.float64, device="cuda")
+    ss, es = (1, batch) if layout == "element-major" else (width, 1)
+    ptr = [v.data_ptr() for v in dev]
+    qa.check(qa.lib().qz_tridiag_thomas_batched(*ptr, x.data_ptr(), M, batch, ss, es, work.data_ptr(), None))
+    torch.cuda.synchronize()
+    got = x.cpu().numpy()
+    got = got.T if layout == "element-major" else got[:, :M]
+    for s in range(n):
+        r, g = np.asarray(ref[s]), np.ascontiguousarray(got[s])
+        nan = np.isnan(r)
+        assert np.array_equal(np.isnan(g), nan), s
+        assert np.array_equal(g[~nan].view(np.int64), r[~nan].view(np.int64)), s
+
+
 @pytest.mark.parametrize("N", [769, 1024])
 def test_rows_large_m0(qa, oracle, decks, N):
     ov = {"grid.rmax": 8, "grid.dr": 8.0 / N, "xi.min": -0.9, "xi.step": 0.03, "driver.n0": 1.5, "driver.sigma_r": 0.4,
