@@ -44,12 +44,13 @@ __device__ __forceinline__ Real dpp_rol(Real src) {
     return __hiloint2double(hi, lo);
 }
 
-// 1 / d by the hardware's estimate (a relative error of at most 2^-24) and two Newton steps: the correctly rounded value
-// but for about one operand in 2^42, and at the ends of the exponent range
+// 1 / d by the hardware's estimate (a relative error of at most 2^-24) and one third-order step: the correctly rounded
+// value but for about one operand in 2^19, and at the ends of the exponent range.  Its users compare every result with
+// the division.
 __device__ __forceinline__ Real chain_recip(Real d) {
-    const Real y0 = __builtin_amdgcn_rcp(d);
-    const Real y1 = __builtin_fma(__builtin_fma(-d, y0, Real(1)), y0, y0);
-    return __builtin_fma(__builtin_fma(-d, y1, Real(1)), y1, y1);
+    const Real y = __builtin_amdgcn_rcp(d);
+    const Real e = __builtin_fma(-d, y, Real(1));
+    return __builtin_fma(__builtin_fma(e, e, e), y, y);
 }
 
 // rows i .. i + R - 1 (i even) of an LDS array of M values padded to an even count and aligned to 16 bytes; rows from
@@ -78,14 +79,15 @@ template <int R> __device__ __forceinline__ void chain_store(Real* p, int i, int
 // without one repeats another's, and writes the same values).
 // Measured (both directions, one wave alone): 513 rows 9.0 us, 257 rows 5.1 us, 65 rows 1.9 us, where one lane per
 // system walking the rows through LDS took 23, 12.6 and 3.8 us.  More rows per lane (16) took no less.
+template <int R = kChainR>
 __device__ __forceinline__ void thomas_wave(const Real* a, const Real* m, const Real* cp, Real b0, Real* w, Real* x,
                                             Real scale, bool dir0, bool dirN, bool fluxN, Real fcw, int M) {
-    constexpr int R = kChainR;
+    constexpr int kBlock = 16 * R;
     const int N = M - 1, l = threadIdx.x & 15;
-    const int nb = (M + kChainBlock - 1) / kChainBlock;
+    const int nb = (M + kBlock - 1) / kBlock;
     Real carry = Real(0);   // dp of the row before the block, in its first lane
     for (int b = 0; b < nb; ++b) {
-        const int i0 = b * kChainBlock + l * R;
+        const int i0 = b * kBlock + l * R;
         Real d[R], av[R], mv[R], pv[R];
         chain_load<R>(w, i0, M, d);
         chain_load<R>(a, i0, M, av);
@@ -107,7 +109,7 @@ __device__ __forceinline__ void thomas_wave(const Real* a, const Real* m, const 
                 if (i0 + r > N) d[r] = av[r] = mv[r] = Real(0);
             }
         }
-        const int steps = min(16, (M - b * kChainBlock + R - 1) / R);
+        const int steps = min(16, (M - b * kBlock + R - 1) / R);
         Real q = carry;
         pv[R - 1] = Real(0);
         for (int s = 0; s < steps; s += 4) {
@@ -127,7 +129,7 @@ __device__ __forceinline__ void thomas_wave(const Real* a, const Real* m, const 
     }
     carry = Real(0);   // x of the row after the block, in its last lane
     for (int b = nb - 1; b >= 0; --b) {
-        const int i0 = b * kChainBlock + l * R;
+        const int i0 = b * kBlock + l * R;
         Real pv[R], cv[R], xv[R];
         chain_load<R>(w, i0, M, pv);
         chain_load<R>(cp, i0, M, cv);
@@ -141,7 +143,7 @@ __device__ __forceinline__ void thomas_wave(const Real* a, const Real* m, const 
         // the rows' values reach the last block's used lanes from lanes that hold zeros
         Real q = carry;
         xv[0] = Real(0);
-        const int steps = min(16, (M - b * kChainBlock + R - 1) / R);
+        const int steps = min(16, (M - b * kBlock + R - 1) / R);
         for (int s = 0; s < steps; s += 4) {
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
@@ -166,16 +168,17 @@ __device__ __forceinline__ void thomas_wave(const Real* a, const Real* m, const 
 // The reciprocal in the chain is chain_recip; after its steps a block is divided once more with the IEEE division, all
 // its rows at once, and one with any difference is run again with that division in the chain.
 // Measured: 513 rows 16.8 us, 257 rows 9.1 us, where one lane per system dividing in the chain took 48 and 23 us.
+template <int R = kChainR>
 __device__ __forceinline__ Real thomas_factor_wave(const Real* a, const Real* b, const Real* c, const Real* chi, Real aN,
                                                    Real bN, bool dir0, bool dirN, Real* __restrict__ m,
                                                    Real* __restrict__ cp, int M) {
-    constexpr int R = kChainR;
+    constexpr int kBlock = 16 * R;
     const int N = M - 1, l = threadIdx.x & 15;
-    const int nb = (M + kChainBlock - 1) / kChainBlock;
+    const int nb = (M + kBlock - 1) / kBlock;
     const Real bw0 = dir0 ? b[0] : b[0] - chi[0];
     Real carry = Real(0);
     for (int k = 0; k < nb; ++k) {
-        const int i0 = k * kChainBlock + l * R;
+        const int i0 = k * kBlock + l * R;
         Real w[R], av[R], cv[R], mv[R], pv[R];
         chain_load<R>(b, i0, M, w);
         chain_load<R>(chi, i0, M, av);
@@ -201,7 +204,7 @@ __device__ __forceinline__ Real thomas_factor_wave(const Real* a, const Real* b,
                 }
             }
         }
-        const int steps = min(16, (M - k * kChainBlock + R - 1) / R);
+        const int steps = min(16, (M - k * kBlock + R - 1) / R);
         auto rows = [&](Real p, auto recip) {
 #pragma unroll
             for (int r = 0; r < R; ++r) {

@@ -12,7 +12,9 @@ __global__ __launch_bounds__(kBS) void sweep_kernel(const qz_sweep_args* __restr
     sweep_run<M1, PT>(runs[blockIdx.x]);
 }
 
-// LDS bytes the kernel needs for N cells, PT particles per thread and L live particles
+// LDS bytes of the runs that the one-workgroup sweep takes: N cells, PT particles per thread, L live particles.  The
+// sort's arrays are counted beside the region they share with the lists: that room (its counters alone take 16 N bytes)
+// holds the lists' shifts (8 (N + 1) bytes).
 long sweep_lds_needed(bool m1, int N, int pt, int L) {
     const LdsPlan plan(N, pt);
     const long Mp = plan.Mp;
@@ -21,7 +23,7 @@ long sweep_lds_needed(bool m1, int N, int pt, int L) {
     long need = nmax * Mp;
     need = std::max(need, nsdep * Mp + 2L * L);   // staged fields + one S+ contribution list
     need = std::max(need, 2L * L);                // one deposit contribution list
-    return plan.region + need * 8;
+    return plan.region + plan.sort + need * 8;
 }
 
 }  // namespace qz

@@ -155,6 +155,40 @@ __device__ __forceinline__ Real sum_list(const Real* v, int e0, int e1) {
     return acc;
 }
 
+// the same sums of two lists of one range, the second `off` doubles after the first (off = 0: the first again); kDeep: 16
+// entries of each in flight (64 registers), else 8
+template <bool kDeep>
+__device__ __forceinline__ void sum_lists(const Real* v, int off, int e0, int e1, Real& x, Real& y) {
+    Real ax = Real(0), ay = Real(0);
+    int e = e0;
+    const Real* w = v + off;
+    if constexpr (kDeep)
+        for (; e + 16 <= e1; e += 16) {
+            Batch8 a, b, c, d;
+            a.load(v + e); b.load(w + e); c.load(v + e + 8); d.load(w + e + 8);
+            a.add_to(ax); b.add_to(ay); c.add_to(ax); d.add_to(ay);
+        }
+    for (; e + 8 <= e1; e += 8) {
+        Batch8 a, b;
+        a.load(v + e); b.load(w + e);
+        a.add_to(ax); b.add_to(ay);
+    }
+    if (e + 4 <= e1) {
+        const Real a0 = v[e], a1 = v[e + 1], a2 = v[e + 2], a3 = v[e + 3];
+        const Real b0 = w[e], b1 = w[e + 1], b2 = w[e + 2], b3 = w[e + 3];
+        ax += a0; ax += a1; ax += a2; ax += a3;
+        ay += b0; ay += b1; ay += b2; ay += b3;
+        e += 4;
+    }
+    for (; e < e1; ++e) {
+        const Real a0 = v[e], b0 = w[e];
+        ax += a0;
+        ay += b0;
+    }
+    x = ax;
+    y = ay;
+}
+
 // entries < key in the index-sorted range idx[lo, hi)
 __device__ __forceinline__ int count_less(const unsigned short* __restrict__ idx, int lo, int hi, int key) {
     int a = lo, b = hi;
@@ -170,6 +204,25 @@ __device__ __forceinline__ int count_less(const unsigned short* __restrict__ idx
 template <class T, int PT> __device__ __forceinline__ void fence_regs(T (&a)[PT]) {
 #pragma unroll
     for (int i = 0; i < PT; ++i) asm volatile("" : "+v"(a[i]));
+}
+
+// f(IC<0>) ... f(IC<n - 1>)
+template <int n, int i = 0, class F> __device__ __forceinline__ void for_each_batch(F&& f) {
+    if constexpr (i < n) {
+        f(IC<i>{});
+        for_each_batch<n, i + 1>(f);
+    }
+}
+
+// grid_weights with the cell searched from `near`: a particle moves by a cell or less in most slices, and the cell and
+// its neighbours' four nodes cost one LDS round trip where the bisection costs one per level
+__device__ __forceinline__ void grid_weights_near(const Real* __restrict__ r, const Real* __restrict__ inv_h, int N, Real R,
+                                                  Real x, int near, int& j, Real& t) {
+    const Real a = r[max(near - 1, 0)], b = r[near], c = r[near + 1], d = r[min(near + 2, N)];
+    if (x > Real(0) && x < R && a <= x && x < d) j = x < b ? near - 1 : (x < c ? near : near + 1);
+    else j = grid_locate(r, N, R, x);
+    t = (x - r[j]) * inv_h[j];
+    t = t < Real(0) ? Real(0) : (t > Real(1) ? Real(1) : t);
 }
 
 __device__ __forceinline__ Real lin(const Real* f, int j, Real t) { return (Real(1) - t) * f[j] + t * f[j + 1]; }

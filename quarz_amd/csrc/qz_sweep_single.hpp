@@ -33,17 +33,19 @@ constexpr int kNW = kBS / 64;      // waves per run
 constexpr int kLdsBytes = 160 * 1024;
 constexpr int kMiscBytes = 512;    // counters, bw0 of the chi factors, deposit component list, phase clocks
 
-// byte offsets of the LDS carve-up: r | 1/h | 1/V | wave counters | cell starts | sorted ids | misc | region
+// byte offsets of the LDS carve-up: r | 1/h | 1/V | cell starts | misc | region.  The sort's wave counters and sorted ids
+// lie at the start of the region: nothing else is in it while the particles are sorted.
 struct LdsPlan {
-    int Mp, wcnt, cs, sidx, misc, region;
+    int Mp, cs, misc, region, wcnt, sidx, sort;
     __host__ __device__ LdsPlan(int N, int pt) {
         const int M = N + 1;
         Mp = (M + 1) & ~1;
-        wcnt = 3 * Mp * 8;
-        cs = wcnt + (((kNW * N * 2) + 15) & ~15);
-        sidx = cs + ((((N + 3) * 4) + 15) & ~15);
-        misc = sidx + (((kBS * pt * 2) + 15) & ~15);
+        cs = 3 * Mp * 8;
+        misc = cs + ((((N + 3) * 4) + 15) & ~15);
         region = misc + kMiscBytes;
+        wcnt = region;
+        sidx = wcnt + (((kNW * N * 2) + 15) & ~15);
+        sort = sidx + (((kBS * pt * 2) + 15) & ~15) - region;   // bytes of the sort's arrays
     }
 };
 
@@ -124,8 +126,6 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
     Real* s_bw0 = reinterpret_cast<Real*>(smem + plan.misc + 16);                        // 4 doubles
     int* s_comp = reinterpret_cast<int*>(smem + plan.misc + 48);                         // 24 ints
     unsigned long long* s_ph = reinterpret_cast<unsigned long long*>(smem + plan.misc + 160);   // phase clocks + last
-    // order of the per-node sums (in the wave-counter area once the sort is done): M node ids
-    unsigned short* s_norder = reinterpret_cast<unsigned short*>(smem + plan.wcnt);
     Real* B = reinterpret_cast<Real*>(smem + plan.region);
     const int Bcap = (kLdsBytes - plan.region) / 8;
     auto BA = [&](int slot) -> Real* { return B + static_cast<size_t>(slot) * Mp; };
@@ -179,10 +179,18 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
     // positions, and the geometry that costs divisions; momenta and weights are re-read where needed
     int cj[PT], cpos[PT];   // cell; node-list positions left | right << 16
     Real ct[PT], cc[PT], cs[PT], cir[PT], cinvd[PT], cgam[PT];
+    // up to 4 particles per thread the momenta, Delta and weight stay in registers for the slice too: every pass over
+    // the particles is then free of loads (a pass's L2 round trip costs more than its arithmetic)
+    constexpr int kRows = PT <= 4 ? kChainR : 4;   // rows per lane of the chains: their registers beside the particles'
+    constexpr bool kMom = PT <= 4;
+    constexpr int PM = kMom ? PT : 1;
+    Real cpx[PM], cpy[PM], cdl[PM], cw[PM];
     auto fence_cache = [&]() {
         fence_regs(cj); fence_regs(cpos); fence_regs(ct); fence_regs(cc); fence_regs(cs); fence_regs(cir);
         fence_regs(cinvd); fence_regs(cgam);
     };
+#pragma unroll
+    for (int pp = 0; pp < PT; ++pp) cj[pp] = 0;   // the last slice's cell: where the search starts
 
     for (int k = kb; k < ke; ++k) {
         // every per-thread value (addresses, lane roles) is formed inside the slice, not kept live across it
@@ -205,46 +213,72 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
         auto load_batch = [&](int p0, Real (&PX)[PB], Real (&PY)[PB], Real (&D)[PB], Real (&wi)[PB]) {
 #pragma unroll
             for (int u = 0; u < PB; ++u) {
-                PX[u] = PY[u] = D[u] = wi[u] = Real(0);
-                if (cj[p0 + u] >= 0) load_mom(p0 + u, PX[u], PY[u], D[u], wi[u]);
+                if constexpr (kMom) {
+                    PX[u] = cpx[p0 + u]; PY[u] = cpy[p0 + u]; D[u] = cdl[p0 + u]; wi[u] = cw[p0 + u];
+                } else {
+                    PX[u] = PY[u] = D[u] = wi[u] = Real(0);
+                    if (cj[p0 + u] >= 0) load_mom(p0 + u, PX[u], PY[u], D[u], wi[u]);
+                }
             }
         };
         // ================================================================ 1. geometry (PlasmaSpecies.cpp:52-70)
+        // the beam sources' next row, first read by this slice's combine, is brought to the cache meanwhile
+        Real ahead[4] = {Real(0), Real(0), Real(0), Real(0)};
+        if (k + 1 < K) {
+            const Real* row = A.bsrc + static_cast<size_t>(k + 1) * M * A.ncb;
 #pragma unroll
-        for (int pp = 0; pp < PT; ++pp) {
-            const int gi = slot_of(pp);
-            cj[pp] = -1;
-            if (gi < NP) {
-                const bool s1 = gi >= np0;
-                const qz_species_state& st = s1 ? A.sp[1] : A.sp[0];
-                const int li = s1 ? gi - np0 : gi;
-                const Real wi = st.w[li];
+            for (int u = 0; u < 4; ++u) ahead[u] = row[min((tid + u * kBS) * 8, M * A.ncb - 1)];
+        }
+        constexpr int PG = PT <= 4 ? PT : 2;
+#pragma unroll
+        for (int p0 = 0; p0 < PT; p0 += PG) {
+            // every load of the batch before the first use
+            Real X[PG], Y[PG], PX[PG], PY[PG], D[PG], wi[PG];
+#pragma unroll
+            for (int u = 0; u < PG; ++u) {
+                const int gi = slot_of(p0 + u);
+                X[u] = Y[u] = PX[u] = PY[u] = D[u] = wi[u] = Real(0);
+                if (gi < NP) {
+                    const bool s1 = gi >= np0;
+                    const qz_species_state& st = s1 ? A.sp[1] : A.sp[0];
+                    const int li = s1 ? gi - np0 : gi;
+                    X[u] = st.x[li]; Y[u] = st.y[li]; PX[u] = st.px[li]; PY[u] = st.py[li]; D[u] = st.dl[li];
+                    wi[u] = st.w[li];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < PG; ++u) {
+                const int pp = p0 + u;
+                const int gi = slot_of(pp);
+                const int hint = max(cj[pp], 0);
+                cj[pp] = -1;
                 // the state at the start of the slice, for the adjoint's recomputation
-                Real* tr = A.traj ? A.traj + static_cast<size_t>(k - kb) * 6 * NP + gi : nullptr;
-                if (tr) tr[5 * static_cast<size_t>(NP)] = wi;
-                if (wi != Real(0)) {
-                    const Real X = st.x[li], Y = st.y[li];
-                    const Real PX = st.px[li], PY = st.py[li], D = st.dl[li];
-                    if (tr) {
-                        tr[0] = X;
-                        tr[NP] = Y;
-                        tr[2 * static_cast<size_t>(NP)] = PX;
-                        tr[3 * static_cast<size_t>(NP)] = PY;
-                        tr[4 * static_cast<size_t>(NP)] = D;
+                if (A.traj && gi < NP) {
+                    Real* tr = A.traj + static_cast<size_t>(k - kb) * 6 * NP + gi;
+                    tr[5 * static_cast<size_t>(NP)] = wi[u];
+                    if (wi[u] != Real(0)) {
+                        tr[0] = X[u];
+                        tr[NP] = Y[u];
+                        tr[2 * static_cast<size_t>(NP)] = PX[u];
+                        tr[3 * static_cast<size_t>(NP)] = PY[u];
+                        tr[4 * static_cast<size_t>(NP)] = D[u];
                     }
-                    const Real r = dsqrt(X * X + Y * Y);
+                }
+                if (wi[u] != Real(0)) {
+                    const Real r = dsqrt(X[u] * X[u] + Y[u] * Y[u]);
                     Real c, s_;
-                    if (r > Real(0)) { c = X / r; s_ = Y / r; } else { c = Real(1); s_ = Real(0); }
+                    if (r > Real(0)) { c = X[u] / r; s_ = Y[u] / r; } else { c = Real(1); s_ = Real(0); }
                     int j; Real t;
-                    grid_weights(s_r, s_ih, N, R, r, j, t);
+                    grid_weights_near(s_r, s_ih, N, R, r, hint, j, t);
                     cj[pp] = j;
                     ct[pp] = t;
                     cc[pp] = c;
                     cs[pp] = s_;
                     cir[pp] = r > Real(0) ? Real(1) / r : Real(0);
-                    const Real gam = (Real(1) + PX * PX + PY * PY + D * D) / (Real(2) * D);
+                    const Real gam = (Real(1) + PX[u] * PX[u] + PY[u] * PY[u] + D[u] * D[u]) / (Real(2) * D[u]);
                     cgam[pp] = gam;
-                    cinvd[pp] = Real(1) / D;
+                    cinvd[pp] = Real(1) / D[u];
+                    if constexpr (kMom) { cpx[pp] = PX[u]; cpy[pp] = PY[u]; cdl[pp] = D[u]; cw[pp] = wi[u]; }
                 }
             }
         }
@@ -310,49 +344,52 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
             }
         }
         __syncthreads();
-        // Order of the per-node sums (m = 1): nodes whose lists exceed twice the mean length (a compressed sheath
-        // holds hundreds of entries) first, then the others, each group in node order.  A wave's item round costs
-        // its longest list, so a thread then sums at most one long list per pass: 3.4% off the c2 sweep (eleven
-        // passes of two components).  In m = 0 (four components, passes of up to eight) it costs more than it
-        // saves (+2.9% on the c5 batch), and the sums keep node order.  Wave 0 builds it while the other waves
-        // search their list positions; it is read after the deposit's first barrier (s_misc[1] = number of long
-        // nodes).
-        if (M1 && w == 0) {
-            const unsigned long long lt_mask = (1ull << lane) - 1ull;
-            const int thr = max(8, (4 * L) / M);
-            int nlong = 0;
-            for (int t0 = 0; t0 < M; t0 += 64) {
-                const int n = t0 + lane;
-                nlong += __popcll(__ballot(n < M && s_cs[n + 2] - s_cs[n] > thr));
-            }
-            int cl = 0, csh = nlong;
-            for (int t0 = 0; nlong > 0 && t0 < M; t0 += 64) {   // no long list: the sums take plain node order
-                const int n = t0 + lane;
-                const bool valid = n < M;
-                const bool lg = valid && s_cs[n + 2] - s_cs[n] > thr;
-                const unsigned long long bl = __ballot(lg), bs = __ballot(valid && !lg);
-                if (lg) s_norder[cl + __popcll(bl & lt_mask)] = static_cast<unsigned short>(n);
-                else if (valid) s_norder[csh + __popcll(bs & lt_mask)] = static_cast<unsigned short>(n);
-                cl += __popcll(bl);
-                csh += __popcll(bs);
-            }
-            if (lane == 0) s_misc[1] = nlong;
-        }
         // node n's list holds cell n-1 (right entries) and cell n (left entries), merged in particle-index order
+        // (the four searches of two particles side by side: each step of one is an LDS round trip)
 #pragma unroll
-        for (int pp = 0; pp < PT; ++pp) {
-            const int j = cj[pp];
-            cpos[pp] = 0;
-            if (j >= 0) {
-                const int gi = slot_of(pp);
-                const int less_m = count_less(s_sidx, s_cs[j], s_cs[j + 1], gi);
-                const int less_p = count_less(s_sidx, s_cs[j + 2], s_cs[j + 3], gi);
-                const int pl = (s_cs[j] + s_cs[j + 1]) + lrank[pp] + less_m;
-                const int pr = (s_cs[j + 1] + s_cs[j + 2]) + lrank[pp] + less_p;
-                cpos[pp] = pl | (pr << 16);
+        for (int p0 = 0; p0 < PT; p0 += 2) {
+            int a[4], b[4], key[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int j = cj[p0 + u];
+                key[u] = slot_of(p0 + u);
+                a[2 * u] = a[2 * u + 1] = b[2 * u] = b[2 * u + 1] = 0;
+                if (j >= 0) {
+                    a[2 * u] = s_cs[j]; b[2 * u] = s_cs[j + 1];
+                    a[2 * u + 1] = s_cs[j + 2]; b[2 * u + 1] = s_cs[j + 3];
+                }
+            }
+            while (a[0] < b[0] || a[1] < b[1] || a[2] < b[2] || a[3] < b[3]) {
+                int mid[4], v[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) mid[q] = (a[q] + b[q]) >> 1;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[q] = s_sidx[mid[q]];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if (a[q] >= b[q]) continue;
+                    if (v[q] < key[q >> 1]) a[q] = mid[q] + 1; else b[q] = mid[q];
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int pp = p0 + u;
+                const int j = cj[pp];
+                cpos[pp] = 0;
+                if (j >= 0) {
+                    const int less_m = a[2 * u] - s_cs[j], less_p = a[2 * u + 1] - s_cs[j + 2];
+                    const int pl = (s_cs[j] + s_cs[j + 1]) + lrank[pp] + less_m + j;
+                    const int pr = (s_cs[j + 1] + s_cs[j + 2]) + lrank[pp] + less_p + j + 1;
+                    cpos[pp] = pl | (pr << 16);
+                }
             }
         }
-        const int G = max(1, min(Bcap / max(2 * L, 1), 8));
+        // node n's list starts n entries late: lists of one length, as undisturbed plasma has (8 or 16 entries), would
+        // otherwise start a whole number of LDS rows apart, and a wave's reads of them, one list per lane, would meet in
+        // 4 of the 64 banks (16 entries apart: 350 cycles per read of a wave, 33 with the shift)
+        const int LS = 2 * L + M;   // a component's lists
+        const int G = max(1, min(Bcap / LS, 8));
+        __syncthreads();   // the lists overwrite the sorted ids
         QZ_PHASE(1);
 
         // ================================================================ 3. deposit (node sums in index order)
@@ -360,32 +397,31 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
         // pass: contributions into LDS lists, a barrier, the per-node sums, a barrier.
         Real* __restrict__ Dg = A.diag + static_cast<size_t>(k) * M * A.ncd;
         const int ncd = A.ncd;
-        // (component, node) of sum item `item` of a pass over gcnt <= 8 components, in the order of s_norder
-        // (plain node order when no list is long); the component count by subtraction, not division
-        auto item_node = [&](int item, int gcnt, int nl, int& g, int& n) {
-            int r = item;
-            g = 0;
-            if (r < gcnt * nl) {
-                while (r >= nl) { r -= nl; ++g; }
-                n = s_norder[r];
-            } else {
-                r -= gcnt * nl;
-                const int ns = M - nl;
-                while (r >= ns) { r -= ns; ++g; }
-                n = nl > 0 ? s_norder[nl + r] : r;
+        // the node sums of gcnt lists from v: out(component of the pass, node, sum).  An item is a node's list in two
+        // components, two chains of adds a thread runs side by side; the wall node's items go to the last threads, whose
+        // lists are short, so that N = 512 cells are one round of the workgroup
+        auto node_sums = [&](const Real* v, int gcnt, auto out) {
+            const int npair = (gcnt + 1) >> 1, nitem = N * npair;
+            auto item = [&](int pr, int n) {
+                const int g = 2 * pr;
+                const int e0 = s_cs[n] + s_cs[n + 1] + n, e1 = s_cs[n + 1] + s_cs[n + 2] + n;
+                Real x, y;
+                sum_lists<(PT <= 2)>(v + g * LS, g + 1 < gcnt ? LS : 0, e0, e1, x, y);
+                out(g, n, x);
+                if (g + 1 < gcnt) out(g + 1, n, y);
+            };
+            for (int i = tid; i < nitem; i += kBS) {
+                int pr = 0, n = i;
+                while (n >= N) { n -= N; ++pr; }
+                item(pr, n);
             }
+            if (kBS - 1 - tid < npair) item(kBS - 1 - tid, N);
         };
         {
             int gcur = 0, c0 = 0;
             auto reduce = [&]() {
                 __syncthreads();
-                const int nl = M1 ? s_misc[1] : 0;
-                for (int item = tid; item < M * gcur; item += kBS) {
-                    int g, n;
-                    item_node(item, gcur, nl, g, n);
-                    const int e0 = s_cs[n] + s_cs[n + 1], e1 = s_cs[n + 1] + s_cs[n + 2];
-                    const Real* vb = B + g * 2 * L;
-                    const Real acc = sum_list(vb, e0, e1);
+                node_sums(B, gcur, [&](int g, int n, Real acc) {
                     const int comp = s_comp[c0 + g];
                     Real* Dn = Dg + static_cast<size_t>(n) * ncd;
                     if (comp == W_NE0) Dn[D_NE0] = acc;
@@ -397,7 +433,7 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
                         const Real bgr0 = A.bg[3 * M + n];
                         Dn[D_NI0] = bgr0 > Real(0) ? acc + bgr0 : acc;
                     } else WS(comp)[n] = acc;
-                }
+                });
                 __syncthreads();
                 QZ_PHASE(3);
                 c0 += gcur;
@@ -406,7 +442,7 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
             // contributions of every cached particle to component C (straight-line over the particles)
             auto comp_pass = [&](auto cst) {
                 constexpr int C = decltype(cst)::value;
-                Real* vb = B + gcur * 2 * L;
+                Real* vb = B + gcur * LS;
                 fence_cache();
 #pragma unroll
                 for (int p0 = 0; p0 < PT; p0 += PB) {
@@ -432,29 +468,75 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
                 QZ_PHASE(2);
                 if (++gcur == G) reduce();
             };
-            comp_pass(IC<W_CHI0>{});
-            comp_pass(IC<W_RHOT0>{});
-            comp_pass(IC<W_DRHO0>{});
-            comp_pass(IC<W_JZ0>{});
-            if (has_neg) comp_pass(IC<W_NE0>{});
-            if (has_pos) comp_pass(IC<W_NI0>{});
-            comp_pass(IC<W_JPR1>{});
-            comp_pass(IC<W_JPI1>{});
-            if (M1) {
-                comp_pass(IC<W_CHI1R>{});
-                comp_pass(IC<W_CHI1I>{});
-                comp_pass(IC<W_RHOT1R>{});
-                comp_pass(IC<W_RHOT1I>{});
-                comp_pass(IC<W_DRHO1R>{});
-                comp_pass(IC<W_DRHO1I>{});
-                comp_pass(IC<W_JZ1R>{});
-                comp_pass(IC<W_JZ1I>{});
-                if (has_neg) { comp_pass(IC<W_NE1R>{}); comp_pass(IC<W_NE1I>{}); }
-                if (has_pos) { comp_pass(IC<W_NI1R>{}); comp_pass(IC<W_NI1I>{}); }
-                comp_pass(IC<W_JPR0>{});
-                comp_pass(IC<W_JPI0>{});
-                comp_pass(IC<W_JPR2>{});
-                comp_pass(IC<W_JPI2>{});
+            // the same for several components in one pass over the particles: most of their terms are common
+            auto group_pass = [&](auto... cst) {
+                constexpr int n = sizeof...(cst);
+                if (gcur + n > G) reduce();
+                Real* vb = B + gcur * LS;
+                fence_cache();
+#pragma unroll
+                for (int p0 = 0; p0 < PT; p0 += PB) {
+                    Real PXb[PB], PYb[PB], Db[PB], wb[PB];
+                    load_batch(p0, PXb, PYb, Db, wb);
+#pragma unroll
+                    for (int u = 0; u < PB; ++u) {
+                        const int pp = p0 + u;
+                        const int j = cj[pp];
+                        if (j < 0) continue;
+                        const Real PX = PXb[u], PY = PYb[u], D = Db[u], wi = wb[u];
+                        const bool s1 = slot_of(pp) >= np0;
+                        const Real q = s1 ? q1 : q0, qm = s1 ? qm1 : qm0;
+                        const int pl = cpos[pp] & 0xffff, pr = cpos[pp] >> 16;
+                        const Real ih = s_ih[j], iv0 = s_iv[j], iv1 = s_iv[j + 1];
+                        const Real pz = cgam[pp] - D;
+                        Real* v = vb;
+                        ((v[pl] = dep_value(decltype(cst)::value, 0, j, ct[pp], cc[pp], cs[pp], cir[pp], cinvd[pp], cgam[pp], PX,
+                                            PY, pz, wi, q, qm, iv0, ih),
+                          v[pr] = dep_value(decltype(cst)::value, 1, j, ct[pp], cc[pp], cs[pp], cir[pp], cinvd[pp], cgam[pp], PX,
+                                            PY, pz, wi, q, qm, iv1, ih),
+                          v += LS),
+                         ...);
+                    }
+                }
+                QZ_PHASE(2);
+                gcur += n;
+                if (gcur >= G) reduce();
+            };
+            // up to 2048 particles on a grid that fits, and in m = 1, two components always have room (G >= 2); a pass of
+            // four is taken where they have
+            if constexpr (!M1 && PT > 4) {
+                comp_pass(IC<W_CHI0>{});
+                comp_pass(IC<W_RHOT0>{});
+                comp_pass(IC<W_DRHO0>{});
+                comp_pass(IC<W_JZ0>{});
+                if (has_neg) comp_pass(IC<W_NE0>{});
+                if (has_pos) comp_pass(IC<W_NI0>{});
+                comp_pass(IC<W_JPR1>{});
+                comp_pass(IC<W_JPI1>{});
+            } else if constexpr (!M1) {
+                if (G >= 4) {
+                    group_pass(IC<W_CHI0>{}, IC<W_RHOT0>{}, IC<W_DRHO0>{}, IC<W_JZ0>{});
+                } else {
+                    group_pass(IC<W_CHI0>{}, IC<W_RHOT0>{});
+                    group_pass(IC<W_DRHO0>{}, IC<W_JZ0>{});
+                }
+                if (has_neg) comp_pass(IC<W_NE0>{});
+                if (has_pos) comp_pass(IC<W_NI0>{});
+                group_pass(IC<W_JPR1>{}, IC<W_JPI1>{});
+            } else {
+                group_pass(IC<W_CHI0>{}, IC<W_RHOT0>{});
+                group_pass(IC<W_DRHO0>{}, IC<W_JZ0>{});
+                if (has_neg) comp_pass(IC<W_NE0>{});
+                if (has_pos) comp_pass(IC<W_NI0>{});
+                group_pass(IC<W_JPR1>{}, IC<W_JPI1>{});
+                group_pass(IC<W_CHI1R>{}, IC<W_CHI1I>{});
+                group_pass(IC<W_RHOT1R>{}, IC<W_RHOT1I>{});
+                group_pass(IC<W_DRHO1R>{}, IC<W_DRHO1I>{});
+                group_pass(IC<W_JZ1R>{}, IC<W_JZ1I>{});
+                if (has_neg) group_pass(IC<W_NE1R>{}, IC<W_NE1I>{});
+                if (has_pos) group_pass(IC<W_NI1R>{}, IC<W_NI1I>{});
+                group_pass(IC<W_JPR0>{}, IC<W_JPI0>{});
+                group_pass(IC<W_JPR2>{}, IC<W_JPI2>{});
             }
             if (gcur > 0) reduce();
         }
@@ -481,6 +563,7 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
             const Real* __restrict__ bs = A.bsrc;
             const Real* __restrict__ bg = A.bg;
             const bool ngp = A.ngp != 0;
+            asm volatile("" ::"v"(ahead[0]), "v"(ahead[1]), "v"(ahead[2]), "v"(ahead[3]));
             auto bb = [&](int kk, int j, int comp) { return bs[(static_cast<size_t>(kk) * M + j) * ncb + comp]; };
             for (int j = tid; j < M; j += kBS) {
                 auto dxi_b = [&](int comp) {
@@ -554,11 +637,11 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
             // psi0, ez0, bz0 (L0);  m1: psi1r, psi1i, ez1r, ez1i, bz1r, bz1i (L1D)
             // (one DPP row per system, waves 0, 2 and 3)
             const int sys = min(lane >> 4, 2);
-            thomas_wave(BA(LY::L0A), BA(LY::L0M), BA(LY::L0CP), A.op_b[OP_L0][0], BA(LY::WPSI0 + sys),
+            thomas_wave<kRows>(BA(LY::L0A), BA(LY::L0M), BA(LY::L0CP), A.op_b[OP_L0][0], BA(LY::WPSI0 + sys),
                         BA(LY::WPSI0 + sys), sys == 2 ? Real(1) : Real(-1), false, true, false, Real(0), M);
         } else if (M1 && (w == 2 || w == 3)) {
             const int sys = 3 * (w - 2) + min(lane >> 4, 2);   // psi1r, psi1i, ez1r | ez1i, bz1r, bz1i
-            thomas_wave(BA(LY::L1A), BA(LY::L1M), BA(LY::L1CP), A.op_b[OP_L1D][0], BA(LY::WPSI1R + sys),
+            thomas_wave<kRows>(BA(LY::L1A), BA(LY::L1M), BA(LY::L1CP), A.op_b[OP_L1D][0], BA(LY::WPSI1R + sys),
                         BA(LY::WPSI1R + sys), sys >= 4 ? Real(1) : Real(-1), true, true, false, Real(0), M);
         } else if (w == 1) {
             // this slice's factors of (L - chi0), one DPP row each: L1D, L1F, m1: L0, L2D
@@ -569,7 +652,7 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
             const int op = f == 0 ? OP_L1D : f == 1 ? OP_L1F : f == 2 ? OP_L0 : OP_L2D;
             const Real aN = A.op_a[op][N], bN = A.op_b[op][N];
             const bool dir0 = op != OP_L0, dirN = op != OP_L1F;
-            s_bw0[f] = thomas_factor_wave(a, b, c, BA(LY::CHI0), aN, bN, dir0, dirN, WS(W_FAC0 + 2 * f),
+            s_bw0[f] = thomas_factor_wave<kRows>(a, b, c, BA(LY::CHI0), aN, bN, dir0, dirN, WS(W_FAC0 + 2 * f),
                                           WS(W_FAC0 + 2 * f + 1), M);
         }
         __syncthreads();
@@ -624,9 +707,9 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
 
         // ================================================================ 5c. S+ deposit (PlasmaSpecies::deposit_S, PlasmaSpecies.cpp:516-558)
         {
-            Real* VB = BA(LY::NSDEP);
-            const int vcap = Bcap - LY::NSDEP * Mp;
-            const int GS = max(1, min(vcap / max(2 * L, 1), nS));
+            // the lists take the staged fields' place once every particle has gathered
+            Real* VB = B;
+            const int GS = max(1, min(Bcap / LS, nS));
             __syncthreads();
             // gather W+, E_z, B_z (PlasmaSpecies.cpp:75-89, without B+) and form the particle's a_x, a_y
             Real cax[PT], cay[PT];
@@ -665,81 +748,78 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
                 cay[pp] = (qm * (gam * Wy - PX * Bz) * invd + fp * sn) * invd - PY * dD * invd * invd;
             }
             }
+            __syncthreads();
             QZ_PHASE(8);
             int gcur = 0, c0 = 0;
             auto reduce = [&]() {
                 __syncthreads();
-                const int nl = M1 ? s_misc[1] : 0;
-                for (int item = tid; item < M * gcur; item += kBS) {
-                    int g, n;
-                    item_node(item, gcur, nl, g, n);
-                    const int e0 = s_cs[n] + s_cs[n + 1], e1 = s_cs[n + 1] + s_cs[n + 2];
-                    const Real* vb = VB + g * 2 * L;
-                    const Real acc = sum_list(vb, e0, e1);
-                    WS(W_SR1 + c0 + g)[n] = acc;
-                }
+                node_sums(VB, gcur, [&](int g, int n, Real acc) { WS(W_SR1 + c0 + g)[n] = acc; });
                 __syncthreads();
                 QZ_PHASE(10);
                 c0 += gcur;
                 gcur = 0;
             };
-            // component SC of S+ (0 r1, 1 i1, 2 r0, 3 i0, 4 r2, 5 i2) for every cached particle
+            // the real and imaginary components of one mode of S+ (first component SC: 0 r1, 2 r0, 4 r2) for every cached
+            // particle, in one pass when both have room
             auto s_pass = [&](auto cst) {
                 constexpr int SC = decltype(cst)::value;
                 constexpr int mode = SC < 2 ? 1 : (SC < 4 ? 0 : 2);
-                Real* vb = VB + gcur * 2 * L;
-                fence_cache();
-                fence_regs(cax); fence_regs(cay);
+                for (int part = GS >= 2 ? 3 : 1; part != 0; part = part == 1 ? 2 : 0) {   // bits: real, imaginary
+                    if (gcur + (part == 3 ? 2 : 1) > GS) reduce();
+                    Real* vr = VB + gcur * LS;
+                    Real* vi = part == 3 ? vr + LS : vr;
+                    fence_cache();
+                    fence_regs(cax); fence_regs(cay);
 #pragma unroll
-                for (int p0 = 0; p0 < PT; p0 += PB) {
-                Real PXb[PB], PYb[PB], Db[PB], wb[PB];
-                load_batch(p0, PXb, PYb, Db, wb);
+                    for (int p0 = 0; p0 < PT; p0 += PB) {
+                        Real PXb[PB], PYb[PB], Db[PB], wb[PB];
+                        load_batch(p0, PXb, PYb, Db, wb);
 #pragma unroll
-                for (int u = 0; u < PB; ++u) {
-                    const int pp = p0 + u;
-                    const int j = cj[pp];
-                    if (j < 0) continue;
-                    const Real PX = PXb[u], PY = PYb[u], wi = wb[u];
-                    const bool s1 = slot_of(pp) >= np0;
-                    const Real qq = s1 ? q1 : q0;
-                    const Real t = ct[pp], c = cc[pp], sn = cs[pp];
-                    const Real invd = cinvd[pp];
-                    const Real ux = PX * invd, uy = PY * invd;
-                    const Real ur = c * ux + sn * uy, uth = c * uy - sn * ux;
-                    const Real ck = mode == 1 ? c : (mode == 0 ? Real(1) : c * c - sn * sn);
-                    const Real sk = mode == 1 ? sn : (mode == 0 ? Real(0) : Real(2) * c * sn);
-                    const Real ax = cax[pp], ay = cay[pp];
-                    const Real wq = wi * qq;
-                    const Real ih = s_ih[j];
-                    const int pl = cpos[pp] & 0xffff, pr = cpos[pp] >> 16;
+                        for (int u = 0; u < PB; ++u) {
+                            const int pp = p0 + u;
+                            const int j = cj[pp];
+                            if (j < 0) continue;
+                            const Real PX = PXb[u], PY = PYb[u], wi = wb[u];
+                            const bool s1 = slot_of(pp) >= np0;
+                            const Real qq = s1 ? q1 : q0;
+                            const Real t = ct[pp], c = cc[pp], sn = cs[pp];
+                            const Real invd = cinvd[pp];
+                            const Real ux = PX * invd, uy = PY * invd;
+                            const Real ur = c * ux + sn * uy, uth = c * uy - sn * ux;
+                            const Real ck = mode == 1 ? c : (mode == 0 ? Real(1) : c * c - sn * sn);
+                            const Real sk = mode == 1 ? sn : (mode == 0 ? Real(0) : Real(2) * c * sn);
+                            const Real ax = cax[pp], ay = cay[pp];
+                            const Real wq = wi * qq;
+                            const Real ih = s_ih[j];
+                            const int pl = cpos[pp] & 0xffff, pr = cpos[pp] >> 16;
 #pragma unroll
-                    for (int side = 0; side < 2; ++side) {
-                        const Real iv = s_iv[j + side] * wq;
-                        const Real W = side == 0 ? Real(1) - t : t;
-                        const Real dW = side == 0 ? -ih : ih;
-                        Real Ar = ax * W + ux * ur * dW;
-                        Real Ai = ay * W + uy * ur * dW;
-                        if (mode != 0) {
-                            const Real Wor = (j == 0) ? (side == 0 ? Real(0) : ih) : W * cir[pp];
-                            const Real f2 = mode * uth * Wor;
-                            Ar += f2 * uy;
-                            Ai -= f2 * ux;
+                            for (int side = 0; side < 2; ++side) {
+                                const Real iv = s_iv[j + side] * wq;
+                                const Real W = side == 0 ? Real(1) - t : t;
+                                const Real dW = side == 0 ? -ih : ih;
+                                Real Ar = ax * W + ux * ur * dW;
+                                Real Ai = ay * W + uy * ur * dW;
+                                if (mode != 0) {
+                                    const Real Wor = (j == 0) ? (side == 0 ? Real(0) : ih) : W * cir[pp];
+                                    const Real f2 = mode * uth * Wor;
+                                    Ar += f2 * uy;
+                                    Ai -= f2 * ux;
+                                }
+                                const int at = side == 0 ? pl : pr;
+                                if (part & 1) vr[at] = iv * (Ar * ck + Ai * sk);
+                                if (part & 2) vi[at] = iv * (Ai * ck - Ar * sk);
+                            }
                         }
-                        const Real v = (SC & 1) == 0 ? iv * (Ar * ck + Ai * sk) : iv * (Ai * ck - Ar * sk);
-                        vb[side == 0 ? pl : pr] = v;
                     }
+                    QZ_PHASE(9);
+                    gcur += part == 3 ? 2 : 1;
+                    if (gcur >= GS) reduce();
                 }
-                }
-                QZ_PHASE(9);
-                if (++gcur == GS) reduce();
             };
             s_pass(IC<0>{});
-            s_pass(IC<1>{});
             if (M1) {
                 s_pass(IC<2>{});
-                s_pass(IC<3>{});
                 s_pass(IC<4>{});
-                s_pass(IC<5>{});
             }
             if (gcur > 0) reduce();
         }
@@ -810,7 +890,7 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
                     const int fidx = sys < 2 ? sys : (sys < 4 ? 2 : 3);   // factor set: L1D, L1F, L0, L2D
                     const Real* a = BA(fidx == 0 ? LY::PA_L1D : fidx == 1 ? LY::PA_L1F : fidx == 2 ? LY::PA_L0 : LY::PA_L2D);
                     const bool flux = fidx == 1;
-                    thomas_wave(a, BA(LY::PF + 2 * fidx), BA(LY::PF + 2 * fidx + 1), s_bw0[fidx], BA(LY::PRB + sys),
+                    thomas_wave<kRows>(a, BA(LY::PF + 2 * fidx), BA(LY::PF + 2 * fidx + 1), s_bw0[fidx], BA(LY::PRB + sys),
                                 BA(LY::PBP + sys), Real(1), fidx != 2, !flux, flux, flux ? fcw : Real(0), M);
                 }
             }
@@ -865,9 +945,35 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
             // ---- Adams-Bashforth push (PlasmaSpecies::push, src/PlasmaSpecies.cpp:600-667)
             const int slot = k % ord;
             const bool first = (k == 0);
+            const int older = first ? 0 : ord;   // slots of the history to read, this one's included
             fence_cache();
+            constexpr int PP = PT == 2 ? 2 : 1;   // particles whose state and history are loaded together
+            for_each_batch<PT / PP>([&](auto batch) {
+            constexpr int p0 = decltype(batch)::value * PP;
+            Real Xb[PP], Yb[PP], Db[PP], PXb[PP], PYb[PP], Hb[PP][4][5];
 #pragma unroll
-            for (int pp = 0; pp < PT; ++pp) {
+            for (int u = 0; u < PP; ++u) {
+                Xb[u] = Yb[u] = Db[u] = PXb[u] = PYb[u] = Real(0);
+                if (cj[p0 + u] >= 0) {
+                    const int gi = slot_of(p0 + u);
+                    const bool s1 = gi >= np0;
+                    const qz_species_state& st = s1 ? A.sp[1] : A.sp[0];
+                    const int li = s1 ? gi - np0 : gi;
+                    Xb[u] = st.x[li]; Yb[u] = st.y[li];
+                    if constexpr (!kMom) { Db[u] = st.dl[li]; PXb[u] = st.px[li]; PYb[u] = st.py[li]; }
+                    const Real* h = st.hist + li;
+#pragma unroll
+                    for (int mm = 1; mm < 5; ++mm)
+                        if (mm < older) {
+                            const int sl = slot - mm + (slot < mm ? ord : 0);
+#pragma unroll
+                            for (int v = 0; v < 5; ++v) Hb[u][mm - 1][v] = h[static_cast<unsigned>((sl * 5 + v) * st.cap)];
+                        }
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < PP; ++u) {
+                const int pp = p0 + u;
                 const int j = cj[pp];
                 if (j < 0) continue;
                 const int gi = slot_of(pp);
@@ -876,8 +982,10 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
                 const int li = s1 ? gi - np0 : gi;
                 const int cap = st.cap;
                 Real* __restrict__ hist = st.hist;
-                const Real X = st.x[li], Y = st.y[li], D = st.dl[li];
-                const Real PX = st.px[li], PY = st.py[li];
+                const Real X = Xb[u], Y = Yb[u];
+                Real D, PX, PY;
+                if constexpr (kMom) { D = cdl[pp]; PX = cpx[pp]; PY = cpy[pp]; }
+                else { D = Db[u]; PX = PXb[u]; PY = PYb[u]; }
                 const Real qm = s1 ? qm1 : qm0;
                 const Real t = ct[pp], c = cc[pp], sn = cs[pp];
                 Real Wx, Wy, Bx, By;
@@ -919,14 +1027,15 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
                     }
                 } else {
                     H(slot, 0) = f0; H(slot, 1) = f1; H(slot, 2) = f2; H(slot, 3) = f3; H(slot, 4) = f4;
-                    for (int mm = 0; mm < ord; ++mm) {
-                        const int sl = (slot - mm + ord) % ord;
+#pragma unroll
+                    for (int mm = 0; mm < 5; ++mm) {
+                        if (mm >= ord) continue;
                         const Real cm = A.ab_c[mm];
                         if (mm == 0) {
                             s0 += cm * f0; sm1 += cm * f1; sm2 += cm * f2; sm3 += cm * f3; sm4 += cm * f4;
                         } else {
-                            s0 += cm * H(sl, 0); sm1 += cm * H(sl, 1); sm2 += cm * H(sl, 2); sm3 += cm * H(sl, 3);
-                            sm4 += cm * H(sl, 4);
+                            const Real* h = Hb[u][mm - 1];
+                            s0 += cm * h[0]; sm1 += cm * h[1]; sm2 += cm * h[2]; sm3 += cm * h[3]; sm4 += cm * h[4];
                         }
                     }
                 }
@@ -960,6 +1069,7 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
                 }
                 st.x[li] = xn; st.y[li] = yn; st.px[li] = pxn; st.py[li] = pyn; st.dl[li] = dn;
             }
+            });
         }
         __syncthreads();
         QZ_PHASE(15);
