@@ -119,36 +119,38 @@ struct Batch8 {
     }
 };
 
-__device__ __forceinline__ Real sum_list(const Real* v, int e0, int e1) {
+// a list in global memory, two entries per load (of any double's address): a wave's lists lie in lines of their own, so
+// its reads cost their count
+typedef double Pair8 __attribute__((ext_vector_type(2), aligned(8)));
+__device__ __forceinline__ Real sum_list_pairs(const Real* v, int e0, int e1) {
     Real acc = Real(0);
     int e = e0;
-    // 24 entries per iteration, all loads issued before the adds: the adds of the first batch cover the
-    // latency of the other two, leaving one exposed LDS round trip per 24 entries
-    for (; e + 24 <= e1; e += 24) {
-        Batch8 x, y, z;
-        x.load(v + e);
-        y.load(v + e + 8);
-        z.load(v + e + 16);
-        x.add_to(acc);
-        y.add_to(acc);
-        z.add_to(acc);
+    for (; e + 32 <= e1; e += 32) {   // all loads of 32 entries in flight: each is a trip to another die's data
+        Pair8 p[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) p[u] = *reinterpret_cast<const Pair8*>(v + e + 2 * u);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) { acc += p[u].x; acc += p[u].y; }
     }
     if (e + 16 <= e1) {
-        Batch8 x, y;
-        x.load(v + e);
-        y.load(v + e + 8);
-        x.add_to(acc);
-        y.add_to(acc);
+        Pair8 p[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) p[u] = *reinterpret_cast<const Pair8*>(v + e + 2 * u);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) { acc += p[u].x; acc += p[u].y; }
         e += 16;
-    } else if (e + 8 <= e1) {
-        Batch8 x;
-        x.load(v + e);
-        x.add_to(acc);
+    }
+    if (e + 8 <= e1) {
+        Pair8 p[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) p[u] = *reinterpret_cast<const Pair8*>(v + e + 2 * u);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) { acc += p[u].x; acc += p[u].y; }
         e += 8;
     }
     if (e + 4 <= e1) {
-        const Real x0 = v[e], x1 = v[e + 1], x2 = v[e + 2], x3 = v[e + 3];
-        acc += x0; acc += x1; acc += x2; acc += x3;
+        const Pair8 p = *reinterpret_cast<const Pair8*>(v + e), q = *reinterpret_cast<const Pair8*>(v + e + 2);
+        acc += p.x; acc += p.y; acc += q.x; acc += q.y;
         e += 4;
     }
     for (; e < e1; ++e) acc += v[e];

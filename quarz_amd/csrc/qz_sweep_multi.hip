@@ -15,11 +15,12 @@ __global__ __launch_bounds__(mBS) void sweep_multi_kernel(const qz_sweep_args* _
     sweep_multi_run<M1, PT>(runs, block_map, static_cast<int>(blockIdx.x));
 }
 
-// LDS bytes of the multi-workgroup kernel for N cells and PT particles per thread
+// LDS bytes of the runs that the multi-workgroup kernel takes, for N cells and PT particles per thread.  The sort's arrays
+// are counted beside the region they share.
 long sweep_multi_lds_needed(bool m1, int N, int pt) {
     const MLds plan(N, pt);
     const long nreg = m1 ? MSlots<true>::NREGION : MSlots<false>::NREGION;
-    return plan.region + nreg * plan.Mp * 8;
+    return plan.region + plan.sort + nreg * plan.Mp * 8;
 }
 
 }  // namespace qz

@@ -15,8 +15,8 @@
 //   4. the solves: the psi / E_z / B_z systems of L0, those of L1D (m = 1) and the chi-dependent Thomas factors
 //      of the B+ operators are three jobs for three workgroups, each staging its operators in its own LDS and
 //      running its chains in one wave (qz_chain.hpp) (grid barrier);
-//   5. every workgroup forms W+ from psi and stages W+, E_z, B_z in LDS; the owned particles gather them and
-//      write their S+ contributions (grid barrier); the node sums of S+ as in 3 (grid barrier);
+//   5. every workgroup forms W+ from psi and stages W+, E_z, B_z in LDS; the owned particles gather them, keep the
+//      gathered values in the workspace for the push and write their S+ contributions (grid barrier); the node sums of S+ as in 3 (grid barrier);
 //   6. the Picard iterations of B+: the systems of each operator pair are one job per workgroup, reading the
 //      previous iterate of the coupled modes from global memory and writing the next one to the other of two
 //      buffers (one grid barrier per iteration);
@@ -47,31 +47,35 @@ constexpr int mLds = 160 * 1024;      // LDS bytes per workgroup
 constexpr int kDepComps = 24;         // deposit arrays (WsArr ids 0 .. 23)
 constexpr unsigned long long kBarrierTicks = 200000000ull;   // 2 s of the 100 MHz wall clock
 
-// layout of the multi-workgroup workspace of a run (doubles): misc | counts | lists | Picard second buffer
+// layout of the multi-workgroup workspace of a run (doubles): misc | counts | lists | Picard second buffer | the fields
+// every particle gathered for S+ (W+ x, y, E_z, B_z), which its push takes again
 struct MwsLayout {
-    size_t misc = 0, cnt, lists, bpalt, total;
+    size_t misc = 0, cnt, lists, bpalt, gath, total;
     __host__ __device__ MwsLayout(int M, int N, int np, int G, bool m1) {
         cnt = 64;   // words 0 barrier, 1 exit count, 2 error; doubles [8..12) bw0
         lists = cnt + (static_cast<size_t>(G) * (N + 1) + 1) / 2 + 1;     // G x N ints
         bpalt = lists + static_cast<size_t>(kDepComps) * 2 * (np > 1 ? np : 1);
-        total = bpalt + static_cast<size_t>(m1 ? 6 : 2) * M;
+        gath = bpalt + static_cast<size_t>(m1 ? 6 : 2) * M;
+        total = gath + 4 * static_cast<size_t>(np);
     }
 };
 
-// LDS carve-up (bytes): r | 1/h | 1/V | wave counters | local cell starts | global cell starts | own offsets |
-// local sorted slots | misc (flags, counts, the deposit array list) | region (Mp-double slots)
+// LDS carve-up (bytes): r | 1/h | 1/V | local cell starts | global cell starts | own offsets | misc (flags, counts, the
+// deposit array list) | region (Mp-double slots).  The sort's wave counters and sorted slots lie at the start of the
+// region: nothing else is in it while the particles are sorted.
 struct MLds {
-    int Mp, wcnt, cs, gcs, goff, sidx, misc, region;
+    int Mp, wcnt, cs, gcs, goff, sidx, misc, region, sort;
     __host__ __device__ MLds(int N, int pt) {
         const int M = N + 1;
         Mp = (M + 1) & ~1;
-        wcnt = 3 * Mp * 8;
-        cs = wcnt + (((mNW * N * 2) + 15) & ~15);
+        cs = 3 * Mp * 8;
         gcs = cs + ((((N + 3) * 4) + 15) & ~15);
         goff = gcs + ((((N + 3) * 4) + 15) & ~15);
-        sidx = goff + ((((N + 2) * 4) + 15) & ~15);
-        misc = sidx + (((mBS * pt * 2) + 15) & ~15);
+        misc = goff + ((((N + 2) * 4) + 15) & ~15);
         region = misc + 256;
+        wcnt = region;
+        sidx = wcnt + (((mNW * N * 2) + 15) & ~15);
+        sort = sidx + (((mBS * pt * 2) + 15) & ~15) - region;   // bytes of the sort's arrays
     }
 };
 
@@ -86,20 +90,31 @@ template <bool M1> struct MSlots {
 };
 }  // namespace
 
+// Every store of this wave has reached the L2: a workgroup's barrier does not wait for that (its waves share one L1), and
+// the release fence of one wave waits for that wave's own stores alone.
+__device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+
 // Grid barrier of the G workgroups of a run.  `target` counts this workgroup's barriers; the shared counter only
 // grows, so barrier n completes when it reaches n G.  Returns false (and sets the run's error flag) when the
 // others do not arrive in time, or when another workgroup has already given up.
 // One release fence before the arrival and one acquire fence after the wait, with the counter itself relaxed
 // (fence-to-fence synchronisation through the counter's release sequence): on this GPU an agent-scope release
 // writes back the die's whole L2 and an acquire invalidates it, operations every other kernel on the die waits
-// behind, so the barrier issues one of each and none per poll.
+// behind, so the barrier issues them once and none per poll.
 __device__ __forceinline__ bool grid_sync(unsigned int* __restrict__ ctr, unsigned int* __restrict__ err, int G,
                                           unsigned int& target, int* s_ok) {
+    wait_stores();
     __syncthreads();
     target += 1;
     if (threadIdx.x == 0) {
         int ok = 1;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");   // this workgroup's writes before the arrival
+        // A second write-back after the first is done.  With one, and the workgroups of other launches writing back the
+        // same die's L2 at the same time, lines made dirty just before the barrier could still be in this L2 when others
+        // read them: 16 of 20 sequences of 16 steps with three in flight read old list entries.  With two none did in 20,
+        // nor with entries stored through to memory (391 us a slice against 353).  A write-back that runs when a request
+        // arrives may have passed those lines; one that starts after the first has ended has not.
+        asm volatile("buffer_wbl2 sc1\n\ts_waitcnt vmcnt(0)" ::: "memory");
         __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const unsigned int want = target * static_cast<unsigned int>(G);
         const unsigned long long t0 = wall_clock64();
@@ -160,6 +175,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
     int* g_cnt = reinterpret_cast<int*>(mws + mw.cnt);
     Real* __restrict__ g_list = mws + mw.lists;
     const size_t lstride = 2 * static_cast<size_t>(NP > 1 ? NP : 1);
+    Real* __restrict__ g_gath = mws + mw.gath;
     Real* bpbuf[2] = {WS(W_BPR1), mws + mw.bpalt};   // Picard iterates: W_BPR1.. of ws, then the second buffer
     unsigned int nbar = 0;
 
@@ -183,15 +199,14 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
 
     const int tid = threadIdx.x;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int lane = tid & 63;
-    const int gthreads = G * mBS, gtid = grp * mBS + tid;
+    const int gthreads = G * mBS;
     for (int j = tid; j < M; j += mBS) {
         s_r[j] = A.grid.r[j];
         s_iv[j] = A.grid.inv_V[j];
         if (j < N) s_ih[j] = A.grid.inv_h[j];
     }
     if (kb == 0)   // B+ := 0 at the head (Simulation.cpp:705-708); every workgroup its share of the nodes
-        for (int j = gtid; j < M; j += gthreads)
+        for (int j = grp * mBS + tid; j < M; j += gthreads)
             for (int a = 0; a < (M1 ? 6 : 2); ++a) WS(W_BPR1 + a)[j] = Real(0);
     // deposit arrays of this run in a fixed order
     int ncomp = 0;
@@ -224,21 +239,34 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
         __syncthreads();
     }
 
-    int cj[PT], lrank[PT], cpl[PT], cpr[PT];
+    int cj[PT], lrank[PT], cpos[PT];   // cell; rank; positions in this workgroup's own lists, left | right << 16
+    constexpr int kRows = PT <= 4 ? kChainR : 4;   // rows per lane of the chains: their registers beside the particles'
+    constexpr bool kMom = PT <= 2;                 // momenta, Delta and weight in registers for the slice
+    constexpr int PM = kMom ? PT : 1, PB = PT <= 4 ? PT : 2;
+    Real cpx[PM], cpy[PM], cdl[PM], cw[PM];
     Real ct[PT], cc[PT], cs[PT], cir[PT], cinvd[PT], cgam[PT];
-    auto slot_of = [&](int pp) { return w * (PT * 64) + pp * 64 + lane; };   // local slot; particle own0 + slot
     auto species_of = [&](int gi, int& li) -> const qz_species_state& {
         const bool s1 = gi >= np0;
         li = s1 ? gi - np0 : gi;
         return s1 ? A.sp[1] : A.sp[0];
     };
 
+#pragma unroll
+    for (int pp = 0; pp < PT; ++pp) cj[pp] = 0;
     bool alive = true;
     for (int k = kb; k < ke && alive; ++k) {
+        // every per-thread value (addresses, lane roles) is formed inside the slice, not kept live across it
+        int tid_k = threadIdx.x;
+        asm volatile("" : "+v"(tid_k));
+        const int tid = tid_k;
+        const int lane = tid & 63;
+        const int gtid = grp * mBS + tid;
+        auto slot_of = [&](int pp) { return w * (PT * 64) + pp * 64 + lane; };   // local slot; particle own0 + slot
         // ================================================================ 1. geometry and the local sort
 #pragma unroll
         for (int pp = 0; pp < PT; ++pp) {
             const int gi = own0 + slot_of(pp);
+            const int near = max(cj[pp], 0);   // the last slice's cell
             cj[pp] = -1;
             if (gi < NP) {
                 int li;
@@ -251,11 +279,12 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     Real c, s_;
                     if (r > Real(0)) { c = X / r; s_ = Y / r; } else { c = Real(1); s_ = Real(0); }
                     int j; Real t;
-                    grid_weights(s_r, s_ih, N, R, r, j, t);
+                    grid_weights_near(s_r, s_ih, N, R, r, near, j, t);
                     cj[pp] = j; ct[pp] = t; cc[pp] = c; cs[pp] = s_;
                     cir[pp] = r > Real(0) ? Real(1) / r : Real(0);
                     cgam[pp] = (Real(1) + PX * PX + PY * PY + D * D) / (Real(2) * D);
                     cinvd[pp] = Real(1) / D;
+                    if constexpr (kMom) { cpx[pp] = PX; cpy[pp] = PY; cdl[pp] = D; cw[pp] = wi; }
                 }
             }
         }
@@ -339,41 +368,95 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
             if (grp == 0 && A.stats) atomicAdd(A.stats, static_cast<unsigned long long>(Ltot));
         }
         __syncthreads();
-        // positions of the two contributions of every owned particle in the global node lists: node n holds
-        // cell n-1 (right entries) and cell n (left entries), merged in particle-index order
+        // The two contributions of every owned particle get their positions in the run's node lists: node n holds cell
+        // n-1 (right entries) and cell n (left entries), merged in particle-index order, and this workgroup's entries are
+        // one run of it after those of the earlier workgroups.  Of the position only that among the workgroup's own
+        // entries is kept, in 16 bits a side; the offset of the run follows from the cell.  The entries go to memory as
+        // they are formed, all components of a particle in turn: a store of a wave takes a line per lane, but nothing
+        // waits for it.  Gathered in LDS in list order first and copied out coalesced they take longer (m = 1, 32768
+        // particles over 8 workgroups 444 us a slice against 353; 8192 over 4 136.6 against 130).
 #pragma unroll
         for (int pp = 0; pp < PT; ++pp) {
             const int j = cj[pp];
+            cpos[pp] = 0;
             if (j >= 0) {
                 const int sl = slot_of(pp);
-                const int rank = s_goff[j + 1] + lrank[pp];
-                const int less_m = s_goff[j] + count_less(s_sidx, s_cs[j], s_cs[j + 1], sl);
-                const int less_p = s_goff[j + 2] + count_less(s_sidx, s_cs[j + 2], s_cs[j + 3], sl);
-                cpl[pp] = (s_gcs[j] + s_gcs[j + 1]) + rank + less_m;
-                cpr[pp] = (s_gcs[j + 1] + s_gcs[j + 2]) + rank + less_p;
+                const int less_m = count_less(s_sidx, s_cs[j], s_cs[j + 1], sl);
+                const int less_p = count_less(s_sidx, s_cs[j + 2], s_cs[j + 3], sl);
+                const int pl = (s_cs[j] + s_cs[j + 1]) + lrank[pp] + less_m;
+                const int pr = (s_cs[j + 1] + s_cs[j + 2]) + lrank[pp] + less_p;
+                cpos[pp] = pl | (pr << 16);
             }
         }
+        auto shift = [&](int n) {   // own run of node n: from its place in the own lists to that in the run's
+            return (s_gcs[n] + s_gcs[n + 1]) + s_goff[n] + s_goff[n + 1] - (s_cs[n] + s_cs[n + 1]);
+        };
+        __syncthreads();   // the sorted slots are read: staged fields may take their place
+        // momenta, Delta and weight of PB consecutive particles from p0, all loads issued before any is used
+        auto load_batch = [&](int p0, Real (&PX)[PB], Real (&PY)[PB], Real (&D)[PB], Real (&wi)[PB]) {
+#pragma unroll
+            for (int u = 0; u < PB; ++u) {
+                if constexpr (kMom) {
+                    PX[u] = cpx[p0 + u]; PY[u] = cpy[p0 + u]; D[u] = cdl[p0 + u]; wi[u] = cw[p0 + u];
+                } else {
+                    PX[u] = PY[u] = D[u] = wi[u] = Real(0);
+                    if (cj[p0 + u] >= 0) {
+                        int gi = own0 + slot_of(p0 + u), li;
+                        asm volatile("" : "+v"(gi));
+                        const qz_species_state& st = species_of(gi, li);
+                        PX[u] = st.px[li]; PY[u] = st.py[li]; D[u] = st.dl[li]; wi[u] = st.w[li];
+                    }
+                }
+            }
+        };
+        auto fence_cache = [&]() {
+            fence_regs(cj); fence_regs(cpos); fence_regs(ct); fence_regs(cc); fence_regs(cs); fence_regs(cir);
+            fence_regs(cinvd); fence_regs(cgam);
+        };
 
         // ================================================================ 3. deposit: contributions, node sums
+        {
+            fence_cache();
 #pragma unroll
-        for (int pp = 0; pp < PT; ++pp) {
-            const int j = cj[pp];
-            if (j < 0) continue;
-            int li;
-            const int gi = own0 + slot_of(pp);
-            const qz_species_state& st = species_of(gi, li);
-            const bool s1 = gi >= np0;
-            const Real PX = st.px[li], PY = st.py[li], D = st.dl[li], wi = st.w[li];
-            const Real q = s1 ? q1 : q0, qm = s1 ? qm1 : qm0;
-            const Real ih = s_ih[j];
-            const Real pz = cgam[pp] - D;
-            for (int ci = 0; ci < ncomp; ++ci) {
-                Real* L = g_list + static_cast<size_t>(ci) * lstride;
-                const int C = s_comps[ci];
-                L[cpl[pp]] = dep_value(C, 0, j, ct[pp], cc[pp], cs[pp], cir[pp], cinvd[pp], cgam[pp], PX, PY, pz, wi,
-                                       q, qm, s_iv[j], ih);
-                L[cpr[pp]] = dep_value(C, 1, j, ct[pp], cc[pp], cs[pp], cir[pp], cinvd[pp], cgam[pp], PX, PY, pz, wi,
-                                       q, qm, s_iv[j + 1], ih);
+            for (int p0 = 0; p0 < PT; p0 += PB) {
+                Real PXb[PB], PYb[PB], Db[PB], wb[PB];
+                load_batch(p0, PXb, PYb, Db, wb);
+#pragma unroll
+                for (int u = 0; u < PB; ++u) {
+                    const int pp = p0 + u;
+                    const int j = cj[pp];
+                    if (j < 0) continue;
+                    const Real PX = PXb[u], PY = PYb[u], D = Db[u], wi = wb[u];
+                    const bool s1 = own0 + slot_of(pp) >= np0;
+                    const Real q = s1 ? q1 : q0, qm = s1 ? qm1 : qm0;
+                    const int gl = (cpos[pp] & 0xffff) + shift(j), gr = (cpos[pp] >> 16) + shift(j + 1);
+                    const Real ih = s_ih[j], iv0 = s_iv[j], iv1 = s_iv[j + 1];
+                    const Real pz = cgam[pp] - D;
+                    Real* __restrict__ L = g_list;
+                    auto pass = [&](auto... cst) {
+                        ((L[gl] = dep_value(decltype(cst)::value, 0, j, ct[pp], cc[pp], cs[pp], cir[pp], cinvd[pp], cgam[pp], PX,
+                                            PY, pz, wi, q, qm, iv0, ih),
+                          L[gr] = dep_value(decltype(cst)::value, 1, j, ct[pp], cc[pp], cs[pp], cir[pp], cinvd[pp], cgam[pp], PX,
+                                            PY, pz, wi, q, qm, iv1, ih),
+                          L += lstride),
+                         ...);
+                    };
+                    pass(IC<W_CHI0>{}, IC<W_RHOT0>{});
+                    pass(IC<W_DRHO0>{}, IC<W_JZ0>{});
+                    if (has_neg) pass(IC<W_NE0>{});
+                    if (has_pos) pass(IC<W_NI0>{});
+                    pass(IC<W_JPR1>{}, IC<W_JPI1>{});
+                    if constexpr (M1) {
+                        pass(IC<W_CHI1R>{}, IC<W_CHI1I>{});
+                        pass(IC<W_RHOT1R>{}, IC<W_RHOT1I>{});
+                        pass(IC<W_DRHO1R>{}, IC<W_DRHO1I>{});
+                        pass(IC<W_JZ1R>{}, IC<W_JZ1I>{});
+                        if (has_neg) pass(IC<W_NE1R>{}, IC<W_NE1I>{});
+                        if (has_pos) pass(IC<W_NI1R>{}, IC<W_NI1I>{});
+                        pass(IC<W_JPR0>{}, IC<W_JPI0>{});
+                        pass(IC<W_JPR2>{}, IC<W_JPI2>{});
+                    }
+                }
             }
         }
         if (!(alive = grid_sync(bar, err, G, nbar, &s_ok))) break;
@@ -397,7 +480,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
             for (int item = gtid; item < ncomp * M; item += gthreads) {
                 const int ci = item / M, n = item - ci * M;
                 const int e0 = s_gcs[n] + s_gcs[n + 1], e1 = s_gcs[n + 1] + s_gcs[n + 2];
-                const Real acc = sum_list(g_list + static_cast<size_t>(ci) * lstride, e0, e1);
+                const Real acc = sum_list_pairs(g_list + static_cast<size_t>(ci) * lstride, e0, e1);
                 const int comp = s_comps[ci];
                 Real* Dn = Dg + static_cast<size_t>(n) * ncd;
                 // the node sum combined with the background and the beam sources (Simulation.cpp:408-457)
@@ -487,7 +570,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     // psi and E_z: -rhs; B_z: +rhs (FieldSolver::solve scale); L0 keeps the axis row regular
                     const int sys = 3 * w + min(lane >> 4, 2);
                     const bool bz = l0 ? sys == 2 : sys >= 4;
-                    thomas_wave(a, m, cp, A.op_b[op][0], BA(3 + sys), BA(3 + sys), bz ? Real(1) : Real(-1), !l0, true,
+                    thomas_wave<kRows>(a, m, cp, A.op_b[op][0], BA(3 + sys), BA(3 + sys), bz ? Real(1) : Real(-1), !l0, true,
                                 false, Real(0), M);
                 }
                 __syncthreads();
@@ -525,7 +608,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     const int op = f == 0 ? OP_L1D : f == 1 ? OP_L1F : f == 2 ? OP_L0 : OP_L2D;
                     const Real aN = A.op_a[op][N], bN = A.op_b[op][N];
                     const bool dir0 = op != OP_L0, dirN = op != OP_L1F;
-                    g_bw0[f] = thomas_factor_wave(BA(base), BA(base + 1), BA(base + 2), BA(3), aN, bN, dir0, dirN,
+                    g_bw0[f] = thomas_factor_wave<kRows>(BA(base), BA(base + 1), BA(base + 2), BA(3), aN, bN, dir0, dirN,
                                                   WS(W_FAC0 + 2 * f), WS(W_FAC0 + 2 * f + 1), M);
                 }
                 __syncthreads();
@@ -573,61 +656,80 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     Fj[F_BZ1R] = BA(SL::BZ + 1)[j]; Fj[F_BZ1I] = BA(SL::BZ + 2)[j];
                 }
             }
-            // S+ contributions of the owned particles (PlasmaSpecies::deposit_S, PlasmaSpecies.cpp:516-558)
+            // S+ contributions of the owned particles (PlasmaSpecies::deposit_S, PlasmaSpecies.cpp:516-558): the gather of
+            // W+, E_z, B_z and the particle's a_x, a_y, and from these its entries of every component
+            fence_cache();
 #pragma unroll
-            for (int pp = 0; pp < PT; ++pp) {
-                const int j = cj[pp];
-                if (j < 0) continue;
-                int li;
-                const int gi = own0 + slot_of(pp);
-                const qz_species_state& st = species_of(gi, li);
-                const bool s1 = gi >= np0;
-                const Real PX = st.px[li], PY = st.py[li], wi = st.w[li];
-                const Real qm = s1 ? qm1 : qm0, qq = s1 ? q1 : q0;
-                const Real t = ct[pp], c = cc[pp], sn = cs[pp];
-                const Real invd = cinvd[pp];
-                Real Wx, Wy;
-                if (M1)
-                    eval_vector(lin(BA(SL::W + 2), j, t), lin(BA(SL::W + 3), j, t), lin(BA(SL::W + 0), j, t),
-                                lin(BA(SL::W + 1), j, t), lin(BA(SL::W + 4), j, t), lin(BA(SL::W + 5), j, t), c, sn, true,
-                                Wx, Wy);
-                else
-                    eval_vector(Real(0), Real(0), lin(BA(SL::W + 0), j, t), lin(BA(SL::W + 1), j, t), Real(0), Real(0), c,
-                                sn, false, Wx, Wy);
-                const Real Ez = eval_scalar(lin(BA(SL::EZ), j, t), M1 ? lin(BA(SL::EZ + 1), j, t) : Real(0),
-                                            M1 ? lin(BA(SL::EZ + 2), j, t) : Real(0), c, sn, M1);
-                const Real Bz = eval_scalar(lin(BA(SL::BZ), j, t), M1 ? lin(BA(SL::BZ + 1), j, t) : Real(0),
-                                            M1 ? lin(BA(SL::BZ + 2), j, t) : Real(0), c, sn, M1);
-                const Real dA = Real(0);
-                const Real gam = cgam[pp];
-                const Real fp = -Real(0.5) * qm * qm * dA * invd;
-                const Real dD = qm * ((PX * Wx + PY * Wy) * invd - Ez);
-                const Real ax = (qm * (gam * Wx + PY * Bz) * invd + fp * c) * invd - PX * dD * invd * invd;
-                const Real ay = (qm * (gam * Wy - PX * Bz) * invd + fp * sn) * invd - PY * dD * invd * invd;
-                const Real ux = PX * invd, uy = PY * invd;
-                const Real ur = c * ux + sn * uy, uth = c * uy - sn * ux;
-                const Real wq = wi * qq;
-                const Real ih = s_ih[j];
-                for (int SC = 0; SC < nS; ++SC) {
-                    const int mode = SC < 2 ? 1 : (SC < 4 ? 0 : 2);
-                    const Real ck = mode == 1 ? c : (mode == 0 ? Real(1) : c * c - sn * sn);
-                    const Real sk = mode == 1 ? sn : (mode == 0 ? Real(0) : Real(2) * c * sn);
-                    Real* L = g_list + static_cast<size_t>(SC) * lstride;
+            for (int p0 = 0; p0 < PT; p0 += PB) {
+                Real PXb[PB], PYb[PB], Db[PB], wb[PB];
+                load_batch(p0, PXb, PYb, Db, wb);
 #pragma unroll
-                    for (int side = 0; side < 2; ++side) {
-                        const Real iv = s_iv[j + side] * wq;
-                        const Real W = side == 0 ? Real(1) - t : t;
-                        const Real dW = side == 0 ? -ih : ih;
-                        Real Ar = ax * W + ux * ur * dW;
-                        Real Ai = ay * W + uy * ur * dW;
-                        if (mode != 0) {
-                            const Real Wor = (j == 0) ? (side == 0 ? Real(0) : ih) : W * cir[pp];
-                            const Real f2 = mode * uth * Wor;
-                            Ar += f2 * uy;
-                            Ai -= f2 * ux;
+                for (int u = 0; u < PB; ++u) {
+                    const int pp = p0 + u;
+                    const int j = cj[pp];
+                    if (j < 0) continue;
+                    const Real PX = PXb[u], PY = PYb[u], wi = wb[u];
+                    const bool s1 = own0 + slot_of(pp) >= np0;
+                    const Real qq = s1 ? q1 : q0, qm = s1 ? qm1 : qm0;
+                    const Real t = ct[pp], c = cc[pp], sn = cs[pp];
+                    const Real invd = cinvd[pp];
+                    Real Wx, Wy;
+                    if (M1)
+                        eval_vector(lin(BA(SL::W + 2), j, t), lin(BA(SL::W + 3), j, t), lin(BA(SL::W + 0), j, t),
+                                    lin(BA(SL::W + 1), j, t), lin(BA(SL::W + 4), j, t), lin(BA(SL::W + 5), j, t), c, sn, true,
+                                    Wx, Wy);
+                    else
+                        eval_vector(Real(0), Real(0), lin(BA(SL::W + 0), j, t), lin(BA(SL::W + 1), j, t), Real(0), Real(0), c,
+                                    sn, false, Wx, Wy);
+                    const Real Ez = eval_scalar(lin(BA(SL::EZ), j, t), M1 ? lin(BA(SL::EZ + 1), j, t) : Real(0),
+                                                M1 ? lin(BA(SL::EZ + 2), j, t) : Real(0), c, sn, M1);
+                    const Real Bz = eval_scalar(lin(BA(SL::BZ), j, t), M1 ? lin(BA(SL::BZ + 1), j, t) : Real(0),
+                                                M1 ? lin(BA(SL::BZ + 2), j, t) : Real(0), c, sn, M1);
+                    {
+                        Real* gt = g_gath + own0 + slot_of(pp);
+                        gt[0] = Wx;
+                        gt[static_cast<size_t>(NP)] = Wy;
+                        gt[2 * static_cast<size_t>(NP)] = Ez;
+                        gt[3 * static_cast<size_t>(NP)] = Bz;
+                    }
+                    const Real dA = Real(0);
+                    const Real gam = cgam[pp];
+                    const Real fp = -Real(0.5) * qm * qm * dA * invd;
+                    const Real dD = qm * ((PX * Wx + PY * Wy) * invd - Ez);
+                    const Real ax = (qm * (gam * Wx + PY * Bz) * invd + fp * c) * invd - PX * dD * invd * invd;
+                    const Real ay = (qm * (gam * Wy - PX * Bz) * invd + fp * sn) * invd - PY * dD * invd * invd;
+                    const Real ux = PX * invd, uy = PY * invd;
+                    const Real ur = c * ux + sn * uy, uth = c * uy - sn * ux;
+                    const Real wq = wi * qq;
+                    const Real ih = s_ih[j];
+                    Real* __restrict__ L = g_list;
+                    auto s_pass = [&](auto cst) {   // the real and imaginary components of one mode
+                        constexpr int mode = decltype(cst)::value;
+                        const Real ck = mode == 1 ? c : (mode == 0 ? Real(1) : c * c - sn * sn);
+                        const Real sk = mode == 1 ? sn : (mode == 0 ? Real(0) : Real(2) * c * sn);
+#pragma unroll
+                        for (int side = 0; side < 2; ++side) {
+                            const Real iv = s_iv[j + side] * wq;
+                            const Real W = side == 0 ? Real(1) - t : t;
+                            const Real dW = side == 0 ? -ih : ih;
+                            Real Ar = ax * W + ux * ur * dW;
+                            Real Ai = ay * W + uy * ur * dW;
+                            if (mode != 0) {
+                                const Real Wor = (j == 0) ? (side == 0 ? Real(0) : ih) : W * cir[pp];
+                                const Real f2 = mode * uth * Wor;
+                                Ar += f2 * uy;
+                                Ai -= f2 * ux;
+                            }
+                            const int at = (side == 0 ? (cpos[pp] & 0xffff) : (cpos[pp] >> 16)) + shift(j + side);
+                            L[at] = iv * (Ar * ck + Ai * sk);
+                            L[lstride + at] = iv * (Ai * ck - Ar * sk);
                         }
-                        const Real v = (SC & 1) == 0 ? iv * (Ar * ck + Ai * sk) : iv * (Ai * ck - Ar * sk);
-                        L[side == 0 ? cpl[pp] : cpr[pp]] = v;
+                        L += 2 * lstride;
+                    };
+                    s_pass(IC<1>{});
+                    if constexpr (M1) {
+                        s_pass(IC<0>{});
+                        s_pass(IC<2>{});
                     }
                 }
             }
@@ -636,7 +738,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
         for (int item = gtid; item < nS * M; item += gthreads) {
             const int sc = item / M, n = item - sc * M;
             const int e0 = s_gcs[n] + s_gcs[n + 1], e1 = s_gcs[n + 1] + s_gcs[n + 2];
-            WS(W_SR1 + sc)[n] = sum_list(g_list + static_cast<size_t>(sc) * lstride, e0, e1);
+            WS(W_SR1 + sc)[n] = sum_list_pairs(g_list + static_cast<size_t>(sc) * lstride, e0, e1);
         }
         if (!(alive = grid_sync(bar, err, G, nbar, &s_ok))) break;
 
@@ -658,13 +760,19 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     const int fb = job == 0 ? 1 : fa;
                     const int opa = job == 0 ? OP_L1D : (job == 1 ? OP_L0 : OP_L2D);
                     const int opb = job == 0 ? OP_L1F : opa;
+                    // a workgroup with one job keeps its operators, factors and gz (slots 8, 9) over the iterations
+                    const bool staged = it > 0 && G >= njob;
                     for (int j = tid; j < M; j += mBS) {
+                        Real gr, gi;
+                        if (staged) {
+                            gr = BA(8)[j];
+                            gi = BA(9)[j];
+                        } else {
                         BA(0)[j] = A.op_a[opa][j];
                         BA(1)[j] = A.op_a[opb][j];
                         BA(2)[j] = WS(W_FAC0 + 2 * fa)[j]; BA(3)[j] = WS(W_FAC0 + 2 * fa + 1)[j];
                         BA(4)[j] = WS(W_FAC0 + 2 * fb)[j]; BA(5)[j] = WS(W_FAC0 + 2 * fb + 1)[j];
                         // gz: ((d_x + i d_y) J_z)_k + S_k, and the chi_1 coupling with the previous iterate
-                        Real gr, gi;
                         if (job == 0) {
                             const Real t1 = stn.grad(WS(W_JZ0), j);
                             gr = t1 + WS(W_SR1)[j];
@@ -681,6 +789,11 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                                 gr = (t2 - t3) + WS(W_SR2)[j];
                                 gi = (t4 - rh) + WS(W_SI2)[j];
                             }
+                        }
+                        if (M1) {
+                            BA(8)[j] = gr;
+                            BA(9)[j] = gi;
+                        }
                         }
                         Real rr = -gi, ri = gr;
                         if (M1) {
@@ -704,7 +817,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                         const int sys = min(lane >> 4, 1);
                         const int f = sys == 0 ? fa : fb;
                         const bool flux = f == 1;
-                        thomas_wave(BA(sys), BA(2 + 2 * sys), BA(3 + 2 * sys), g_bw0[f], BA(6 + sys), BA(6 + sys),
+                        thomas_wave<kRows>(BA(sys), BA(2 + 2 * sys), BA(3 + 2 * sys), g_bw0[f], BA(6 + sys), BA(6 + sys),
                                     Real(1), f != 2, !flux, flux, flux ? fcw : Real(0), M);
                     }
                     __syncthreads();
@@ -720,17 +833,6 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
         }
 
         // ================================================================ 7. store (Simulation.cpp:594-633) and push
-        // the Picard jobs reused the region: W+, E_z and B_z are staged again for the push gather
-        for (int j = tid; j < M; j += mBS) {
-            for (int a = 0; a < (M1 ? 6 : 2); ++a) BA(SL::W + a)[j] = WS(W_WPR1 + a)[j];
-            BA(SL::EZ)[j] = WS(W_EZ0)[j];
-            BA(SL::BZ)[j] = WS(W_BZ0)[j];
-            if (M1) {
-                BA(SL::EZ + 1)[j] = WS(W_EZ1R)[j]; BA(SL::EZ + 2)[j] = WS(W_EZ1I)[j];
-                BA(SL::BZ + 1)[j] = WS(W_BZ1R)[j]; BA(SL::BZ + 2)[j] = WS(W_BZ1I)[j];
-            }
-        }
-        __syncthreads();
         {
             const Real* bfin = bpbuf[niter & 1];
             auto BF = [&](int f, int j) { return bfin[static_cast<size_t>(f) * M + j]; };
@@ -755,12 +857,43 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     for (int f = 0; f < (M1 ? 6 : 2); ++f) WS(W_BPR1 + f)[j] = BF(f, j);
             }
             if (k < K - 1) {
-                // ---- Adams-Bashforth push (PlasmaSpecies::push, src/PlasmaSpecies.cpp:600-667)
+                // ---- Adams-Bashforth push (PlasmaSpecies::push, src/PlasmaSpecies.cpp:600-667); B+ staged in LDS
                 const int slot = k % ord;
                 const bool first = (k == 0);
-                auto glin = [&](int f, int j, Real t) { return (Real(1) - t) * BF(f, j) + t * BF(f, j + 1); };
+                const int older = first ? 0 : ord;   // slots of the history to read, this one's included
+                for (int j = tid; j < M; j += mBS)
+                    for (int f = 0; f < (M1 ? 6 : 2); ++f) BA(f)[j] = BF(f, j);
+                __syncthreads();
+                fence_cache();
+                constexpr int PP = PT == 2 ? 2 : 1;   // particles whose state and history are loaded together
+                for_each_batch<PT / PP>([&](auto batch) {
+                constexpr int p0 = decltype(batch)::value * PP;
+                Real Xb[PP], Yb[PP], Db[PP], PXb[PP], PYb[PP], Gb[PP][4], Hb[PP][4][5];
 #pragma unroll
-                for (int pp = 0; pp < PT; ++pp) {
+                for (int u = 0; u < PP; ++u) {
+                    Xb[u] = Yb[u] = Db[u] = PXb[u] = PYb[u] = Real(0);
+                    Gb[u][0] = Gb[u][1] = Gb[u][2] = Gb[u][3] = Real(0);
+                    if (cj[p0 + u] >= 0) {
+                        int li;
+                        const int gi = own0 + slot_of(p0 + u);
+                        const qz_species_state& st = species_of(gi, li);
+                        Xb[u] = st.x[li]; Yb[u] = st.y[li];
+                        if constexpr (!kMom) { Db[u] = st.dl[li]; PXb[u] = st.px[li]; PYb[u] = st.py[li]; }
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) Gb[u][v] = g_gath[static_cast<size_t>(v) * NP + gi];
+                        const Real* h = st.hist + li;
+#pragma unroll
+                        for (int mm = 1; mm < 5; ++mm)
+                            if (mm < older) {
+                                const int sl = slot - mm + (slot < mm ? ord : 0);
+#pragma unroll
+                                for (int v = 0; v < 5; ++v) Hb[u][mm - 1][v] = h[static_cast<size_t>(sl * 5 + v) * st.cap];
+                            }
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < PP; ++u) {
+                    const int pp = p0 + u;
                     const int j = cj[pp];
                     if (j < 0) continue;
                     int li;
@@ -769,27 +902,20 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     const qz_species_state& st = species_of(gi, li);
                     const int cap = st.cap;
                     Real* __restrict__ hist = st.hist;
-                    const Real X = st.x[li], Y = st.y[li], D = st.dl[li];
-                    const Real PX = st.px[li], PY = st.py[li];
+                    const Real X = Xb[u], Y = Yb[u];
+                    Real D, PX, PY;
+                    if constexpr (kMom) { D = cdl[pp]; PX = cpx[pp]; PY = cpy[pp]; }
+                    else { D = Db[u]; PX = PXb[u]; PY = PYb[u]; }
                     const Real qm = s1 ? qm1 : qm0;
                     const Real t = ct[pp], c = cc[pp], sn = cs[pp];
-                    Real Wx, Wy, Bx, By;
-                    if (M1) {
-                        eval_vector(lin(BA(SL::W + 2), j, t), lin(BA(SL::W + 3), j, t), lin(BA(SL::W + 0), j, t),
-                                    lin(BA(SL::W + 1), j, t), lin(BA(SL::W + 4), j, t), lin(BA(SL::W + 5), j, t), c, sn,
-                                    true, Wx, Wy);
-                        eval_vector(glin(2, j, t), glin(3, j, t), glin(0, j, t), glin(1, j, t), glin(4, j, t),
-                                    glin(5, j, t), c, sn, true, Bx, By);
-                    } else {
-                        eval_vector(Real(0), Real(0), lin(BA(SL::W + 0), j, t), lin(BA(SL::W + 1), j, t), Real(0),
-                                    Real(0), c, sn, false, Wx, Wy);
-                        eval_vector(Real(0), Real(0), glin(0, j, t), glin(1, j, t), Real(0), Real(0), c, sn, false, Bx,
+                    const Real Wx = Gb[u][0], Wy = Gb[u][1], Ez = Gb[u][2], Bz = Gb[u][3];
+                    Real Bx, By;
+                    if (M1)
+                        eval_vector(lin(BA(2), j, t), lin(BA(3), j, t), lin(BA(0), j, t), lin(BA(1), j, t), lin(BA(4), j, t),
+                                    lin(BA(5), j, t), c, sn, true, Bx, By);
+                    else
+                        eval_vector(Real(0), Real(0), lin(BA(0), j, t), lin(BA(1), j, t), Real(0), Real(0), c, sn, false, Bx,
                                     By);
-                    }
-                    const Real Ez = eval_scalar(lin(BA(SL::EZ), j, t), M1 ? lin(BA(SL::EZ + 1), j, t) : Real(0),
-                                                M1 ? lin(BA(SL::EZ + 2), j, t) : Real(0), c, sn, M1);
-                    const Real Bz = eval_scalar(lin(BA(SL::BZ), j, t), M1 ? lin(BA(SL::BZ + 1), j, t) : Real(0),
-                                                M1 ? lin(BA(SL::BZ + 2), j, t) : Real(0), c, sn, M1);
                     const Real dA = Real(0);
                     const Real gam = cgam[pp];
                     const Real invd = cinvd[pp];
@@ -811,14 +937,15 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                         }
                     } else {
                         H(slot, 0) = f0; H(slot, 1) = f1; H(slot, 2) = f2; H(slot, 3) = f3; H(slot, 4) = f4;
-                        for (int mm = 0; mm < ord; ++mm) {
-                            const int sl = (slot - mm + ord) % ord;
+#pragma unroll
+                        for (int mm = 0; mm < 5; ++mm) {
+                            if (mm >= ord) continue;
                             const Real cm = A.ab_c[mm];
                             if (mm == 0) {
                                 s0 += cm * f0; sm1 += cm * f1; sm2 += cm * f2; sm3 += cm * f3; sm4 += cm * f4;
                             } else {
-                                s0 += cm * H(sl, 0); sm1 += cm * H(sl, 1); sm2 += cm * H(sl, 2); sm3 += cm * H(sl, 3);
-                                sm4 += cm * H(sl, 4);
+                                const Real* h = Hb[u][mm - 1];
+                                s0 += cm * h[0]; sm1 += cm * h[1]; sm2 += cm * h[2]; sm3 += cm * h[3]; sm4 += cm * h[4];
                             }
                         }
                     }
@@ -852,6 +979,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     }
                     st.x[li] = xn; st.y[li] = yn; st.px[li] = pxn; st.py[li] = pyn; st.dl[li] = dn;
                 }
+                });
             }
         }
         __syncthreads();

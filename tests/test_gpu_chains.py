@@ -80,3 +80,21 @@ def test_rows_large_m0(qa, oracle, decks, N):
         g.step()
         o.step()
         assert np.array_equal(g.fld, o.fld) and np.array_equal(g.diag, o.diag), groups
+
+
+def test_steps_in_flight_of_several_workgroups(qa, tmp_path):
+    """Sixteen steps with three in flight, each sweep on eight workgroups beside the others', equal the same steps one at
+    a time, bit for bit: a workgroup reads nothing that another has not yet made visible, whatever runs beside it."""
+    from quarz_amd import configs
+    deck = configs.c3_deck(workdir=str(tmp_path), xi_min=-1.5, steps=30, nd=100000, nw=20000, driver_xi0=-0.6,
+                           witness_xi0=-1.2)
+    ov = {"driver.sigma_xi": 0.2, "driver.x0": 0.05, "driver.n0": 2, "witness.sigma_xi": 0.05}
+    a = qa.Simulation(deck, ov)
+    b = qa.Simulation(deck, ov)
+    assert a.groups == 8 and b.groups == 8
+    for _ in range(16):
+        a.step()
+    b.step()
+    b.run_pipelined(15, chunks=6, depth=3)
+    for w in ("fld", "diag", "bsrc"):
+        assert np.array_equal(np.array(getattr(b, w)), np.array(getattr(a, w))), w
