@@ -164,14 +164,14 @@ __device__ __forceinline__ void thomas_wave(const Real* a, const Real* m, const 
 // Thomas factors of (L - chi) with the Dirichlet rows of FieldSolver::solve (src/FieldSolver.cpp:253-256):
 //   bw_i = b_i (Dirichlet row) or b_i - chi_i;  c'_0 = c_0 / bw_0;  m_i = 1 / (bw_i - a_i c'_{i-1});  c'_i = c_i m_i
 // Rows 0 .. N-1 from a, b, c (LDS); the last row's a_N, b_N given (the flux and Dirichlet variants of L_1
-// share every other row).  m, c' go to global memory.  Returns bw_0.  Called as thomas_wave.
+// share every other row).  put(i, m_i, c'_i) takes every row, from the lane that holds it.  Returns bw_0.  Called as
+// thomas_wave.
 // The reciprocal in the chain is chain_recip; after its steps a block is divided once more with the IEEE division, all
 // its rows at once, and one with any difference is run again with that division in the chain.
 // Measured: 513 rows 16.8 us, 257 rows 9.1 us, where one lane per system dividing in the chain took 48 and 23 us.
-template <int R = kChainR>
+template <int R = kChainR, class Put>
 __device__ __forceinline__ Real thomas_factor_wave(const Real* a, const Real* b, const Real* c, const Real* chi, Real aN,
-                                                   Real bN, bool dir0, bool dirN, Real* __restrict__ m,
-                                                   Real* __restrict__ cp, int M) {
+                                                   Real bN, bool dir0, bool dirN, int M, Put put) {
     constexpr int kBlock = 16 * R;
     const int N = M - 1, l = threadIdx.x & 15;
     const int nb = (M + kBlock - 1) / kBlock;
@@ -244,10 +244,7 @@ __device__ __forceinline__ Real thomas_factor_wave(const Real* a, const Real* b,
         }
 #pragma unroll
         for (int r = 0; r < R; ++r)
-            if (i0 + r < M) {
-                m[i0 + r] = i0 + r == 0 ? Real(0) : mv[r];
-                cp[i0 + r] = pv[r];
-            }
+            if (i0 + r < M) put(i0 + r, i0 + r == 0 ? Real(0) : mv[r], pv[r]);
         carry = dpp_ror(pv[R - 1]);
     }
     return bw0;

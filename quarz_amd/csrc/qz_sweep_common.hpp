@@ -119,42 +119,30 @@ struct Batch8 {
     }
 };
 
-// a list in global memory, two entries per load (of any double's address): a wave's lists lie in lines of their own, so
-// its reads cost their count
-typedef double Pair8 __attribute__((ext_vector_type(2), aligned(8)));
-__device__ __forceinline__ Real sum_list_pairs(const Real* v, int e0, int e1) {
-    Real acc = Real(0);
+// the same sums of a list of rows of S doubles in global memory: of the row's doubles 0, 8, 16 ... (P of them), side by
+// side.  U P loads in flight, each a trip to another die's data.
+template <int S, int P, int U> __device__ __forceinline__ void sum_rows(const Real* v, int e0, int e1, Real (&acc)[P]) {
     int e = e0;
-    for (; e + 32 <= e1; e += 32) {   // all loads of 32 entries in flight: each is a trip to another die's data
-        Pair8 p[16];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) p[u] = *reinterpret_cast<const Pair8*>(v + e + 2 * u);
+    for (int c = 0; c < P; ++c) acc[c] = Real(0);
+    auto take = [&](auto count) {
+        constexpr int n = decltype(count)::value;
+        Real p[n][P];
+        const Real* q = v + static_cast<size_t>(e) * S;
 #pragma unroll
-        for (int u = 0; u < 16; ++u) { acc += p[u].x; acc += p[u].y; }
-    }
-    if (e + 16 <= e1) {
-        Pair8 p[8];
+        for (int u = 0; u < n; ++u)
 #pragma unroll
-        for (int u = 0; u < 8; ++u) p[u] = *reinterpret_cast<const Pair8*>(v + e + 2 * u);
+            for (int c = 0; c < P; ++c) p[u][c] = q[u * S + 8 * c];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) { acc += p[u].x; acc += p[u].y; }
-        e += 16;
-    }
-    if (e + 8 <= e1) {
-        Pair8 p[4];
+        for (int u = 0; u < n; ++u)
 #pragma unroll
-        for (int u = 0; u < 4; ++u) p[u] = *reinterpret_cast<const Pair8*>(v + e + 2 * u);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) { acc += p[u].x; acc += p[u].y; }
-        e += 8;
-    }
-    if (e + 4 <= e1) {
-        const Pair8 p = *reinterpret_cast<const Pair8*>(v + e), q = *reinterpret_cast<const Pair8*>(v + e + 2);
-        acc += p.x; acc += p.y; acc += q.x; acc += q.y;
-        e += 4;
-    }
-    for (; e < e1; ++e) acc += v[e];
-    return acc;
+            for (int c = 0; c < P; ++c) acc[c] += p[u][c];
+        e += n;
+    };
+    while (e + U <= e1) take(IC<U>{});
+    if (e + 8 <= e1) take(IC<8>{});
+    if (e + 4 <= e1) take(IC<4>{});
+    while (e < e1) take(IC<1>{});
 }
 
 // the same sums of two lists of one range, the second `off` doubles after the first (off = 0: the first again); kDeep: 16

@@ -9,21 +9,23 @@
 //      all and forms the global cell starts and its own offsets, so that every contribution gets its position in
 //      its node's list in global particle-index order: workgroups hold consecutive index ranges, so the particles
 //      of earlier workgroups come first, and within a workgroup the local sort gives the order;
-//   3. the contributions of every deposit array go to these global lists (grid barrier); one thread per
-//      (node, array), over all workgroups, sums a list sequentially -- the serial atomic_add order -- and adds
-//      the background and beam sources (combine_sources) (grid barrier);
+//   3. the contributions to every deposit array go to these global lists, an entry holding all arrays side by side
+//      (grid barrier); a lane sums one or three arrays of a node's list sequentially -- the serial atomic_add order --
+//      and adds the background and beam sources (combine_sources) (grid barrier);
 //   4. the solves: the psi / E_z / B_z systems of L0, those of L1D (m = 1) and the chi-dependent Thomas factors
 //      of the B+ operators are three jobs for three workgroups, each staging its operators in its own LDS and
 //      running its chains in one wave (qz_chain.hpp) (grid barrier);
 //   5. every workgroup forms W+ from psi and stages W+, E_z, B_z in LDS; the owned particles gather them, keep the
-//      gathered values in the workspace for the push and write their S+ contributions (grid barrier); the node sums of S+ as in 3 (grid barrier);
+//      gathered values in the workspace for the push and write their S+ contributions (grid barrier); the node sums
+//      of S+ as in 3 (grid barrier);
 //   6. the Picard iterations of B+: the systems of each operator pair are one job per workgroup, reading the
 //      previous iterate of the coupled modes from global memory and writing the next one to the other of two
 //      buffers (one grid barrier per iteration);
 //   7. the field store (node ranges per workgroup) and the Adams-Bashforth push of the owned particles.
 // The grid barrier is a counter in the run's workspace that only grows during a launch: barrier n of the launch
-// completes when it reaches n G; the last workgroup to leave the launch puts it back to zero.  Every wait is bounded in time: a barrier not reached within two seconds marks the run's error
-// flag and ends the launch in every workgroup, and the host reports it.  A launch is refused unless all its
+// completes when it reaches n G; the last workgroup to leave the launch puts it back to zero.  Every wait is bounded in
+// time: a barrier not reached within two seconds marks the run's error flag and ends the launch in every workgroup, and
+// the host reports it.  Whatever crosses a barrier is stored through to memory (share).  A launch is refused unless all its
 // workgroups (and those of the launches the caller keeps in flight beside it) fit the device together, one per
 // compute unit, so every workgroup is resident.  Arithmetic per term is that of the one-workgroup kernel
 // (qz_sweep.hip), so the result is the serial oracle's bit for bit.
@@ -44,19 +46,22 @@ namespace {
 constexpr int mBS = 512;              // threads per workgroup
 constexpr int mNW = mBS / 64;         // waves per workgroup
 constexpr int mLds = 160 * 1024;      // LDS bytes per workgroup
-constexpr int kDepComps = 24;         // deposit arrays (WsArr ids 0 .. 23)
 constexpr unsigned long long kBarrierTicks = 200000000ull;   // 2 s of the 100 MHz wall clock
 
 // layout of the multi-workgroup workspace of a run (doubles): misc | counts | lists | Picard second buffer | the fields
-// every particle gathered for S+ (W+ x, y, E_z, B_z), which its push takes again
+// every particle gathered for S+ (W+ x, y, E_z, B_z), which its push takes again.  These last are their own workgroup's
+// and stay in its L2, so a cache line lies between them and what the workgroups share, and after them.
+constexpr int kLineDoubles = 16;
+constexpr int kEntrySlots = 24;   // doubles of a list entry in m = 1 (8 in m = 0)
 struct MwsLayout {
     size_t misc = 0, cnt, lists, bpalt, gath, total;
     __host__ __device__ MwsLayout(int M, int N, int np, int G, bool m1) {
         cnt = 64;   // words 0 barrier, 1 exit count, 2 error; doubles [8..12) bw0
         lists = cnt + (static_cast<size_t>(G) * (N + 1) + 1) / 2 + 1;     // G x N ints
-        bpalt = lists + static_cast<size_t>(kDepComps) * 2 * (np > 1 ? np : 1);
-        gath = bpalt + static_cast<size_t>(m1 ? 6 : 2) * M;
-        total = gath + 4 * static_cast<size_t>(np);
+        lists = (lists + kLineDoubles - 1) / kLineDoubles * kLineDoubles;
+        bpalt = lists + static_cast<size_t>(kEntrySlots) * 2 * (np > 1 ? np : 1);
+        gath = bpalt + static_cast<size_t>(m1 ? 6 : 2) * M + kLineDoubles;
+        total = gath + 4 * static_cast<size_t>(np) + kLineDoubles;
     }
 };
 
@@ -87,34 +92,126 @@ template <bool M1> struct MSlots {
     // pairs, two right-hand sides)
     static constexpr int NJOB = M1 ? 10 : 8;
     static constexpr int NREGION = NFIELD > NJOB ? NFIELD : NJOB;
+    // doubles of a list entry: every deposit array of one particle and node side by side, in the order of entry_comp
+    static constexpr int ENTRY = M1 ? kEntrySlots : 8;
+    // and of S+ (r1 i1 r0 i0 r2 i2), and the doubles its entry takes
+    static constexpr int NS = M1 ? 6 : 2, SENTRY = M1 ? 8 : 2;
 };
+__device__ constexpr int entry_comp(int slot) {
+    constexpr int order[kEntrySlots] = {W_CHI0, W_RHOT0, W_DRHO0, W_JZ0, W_NE0, W_NI0, W_JPR1, W_JPI1,
+                                        W_CHI1R, W_CHI1I, W_RHOT1R, W_RHOT1I, W_DRHO1R, W_DRHO1I, W_JZ1R, W_JZ1I,
+                                        W_NE1R, W_NE1I, W_NI1R, W_NI1I, W_JPR0, W_JPI0, W_JPR2, W_JPI2};
+    return order[slot];
+}
+// What becomes of a slot's node sum (combine_sources, Simulation.cpp:408-457): kind | destination << 4 (a WsArr or a
+// DiagComp) | beam source << 12 | background << 20 (in units of M); kKindNone for a species sign the run does not have
+enum SumKind : int { kKindChi = 0, kKindBeam, kKindBackground, kKindDxi, kKindDiag, kKindIons, kKindNone = -1 };
+__device__ __forceinline__ int entry_code(int slot, bool has_neg, bool has_pos) {
+    const int comp = entry_comp(slot);
+    auto code = [](int kind, int dst, int beam = 0, int bg = 0) { return kind | dst << 4 | beam << 12 | bg << 20; };
+    switch (comp) {
+        case W_RHOT0: return code(kKindBackground, comp, B_RT0, 0);
+        case W_RHOT1R: return code(kKindBackground, comp, B_RT1R, 1);
+        case W_RHOT1I: return code(kKindBackground, comp, B_RT1I, 2);
+        case W_DRHO0: return code(kKindDxi, comp, B_RT0);
+        case W_DRHO1R: return code(kKindDxi, comp, B_RT1R);
+        case W_DRHO1I: return code(kKindDxi, comp, B_RT1I);
+        case W_JZ0: return code(kKindBeam, comp, B_JZ0);
+        case W_JZ1R: return code(kKindBeam, comp, B_JZ1R);
+        case W_JZ1I: return code(kKindBeam, comp, B_JZ1I);
+        case W_JPR1: return code(kKindBeam, comp, B_JP1R);
+        case W_JPI1: return code(kKindBeam, comp, B_JP1I);
+        case W_JPR0: return code(kKindBeam, comp, B_JP0R);
+        case W_JPI0: return code(kKindBeam, comp, B_JP0I);
+        case W_JPR2: return code(kKindBeam, comp, B_JP2R);
+        case W_JPI2: return code(kKindBeam, comp, B_JP2I);
+        case W_NE0: return has_neg ? code(kKindDiag, D_NE0) : kKindNone;
+        case W_NE1R: return has_neg ? code(kKindDiag, D_NE1R) : kKindNone;
+        case W_NE1I: return has_neg ? code(kKindDiag, D_NE1I) : kKindNone;
+        case W_NI0: return has_pos ? code(kKindIons, D_NI0, 0, 3) : kKindNone;
+        case W_NI1R: return has_pos ? code(kKindDiag, D_NI1R) : kKindNone;
+        case W_NI1I: return has_pos ? code(kKindDiag, D_NI1I) : kKindNone;
+        default: return code(kKindChi, comp);
+    }
+}
 }  // namespace
 
-// Every store of this wave has reached the L2: a workgroup's barrier does not wait for that (its waves share one L1), and
-// the release fence of one wave waits for that wave's own stores alone.
-__device__ __forceinline__ void wait_stores() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// What one workgroup stores and another reads, and every other value of the arrays that hold such values, goes to memory
+// with an agent-scope store: it is written through this die's L2, so no line of these arrays is ever dirty there.  A
+// reader's acquire then drops its die's copies, and nothing depends on what a write-back of an L2 reaches while the
+// workgroups of other launches use it too.  The arrays are reached through pointers to const, so that a plain store to
+// them does not compile.
+template <class T> __device__ __forceinline__ void share(const T* p, T v) {
+    __hip_atomic_store(const_cast<T*>(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// two doubles `off` bytes into such an array, described by `buf`: a store of 16 bytes at agent scope (sc1).  A
+// written-through store costs its request, so what a lane stores side by side goes in as few as it can.
+typedef unsigned int Word4 __attribute__((ext_vector_type(4)));
+typedef double Pair16 __attribute__((ext_vector_type(2)));
+constexpr int kAgentScope = 16;   // the sc1 bit of a buffer instruction's cache policy
+__device__ __forceinline__ void share_pair(__amdgpu_buffer_rsrc_t buf, unsigned int off, Real x, Real y) {
+    const Pair16 v = {x, y};
+    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(Word4, v), buf, off, 0, kAgentScope);
+}
+// The four lanes of a quad hold 64 bytes of a list entry each (p: four pairs of doubles), which belong at `off`: they exchange
+// them so that every store writes one lane's 64 bytes, side by side, in one request.  Called by all lanes of a wave; a lane
+// without an entry gives kNoEntry.  A workgroup's requests leave at one per four cycles or so, whatever their size: the
+// entries of 4096 particles (m = 1, 8 workgroups) and the wait for them take 53 us a slice, 175 us as 16 bytes per lane.
+constexpr unsigned int kNoEntry = ~0u;   // past every buffer's end
+template <int ctrl> __device__ __forceinline__ Word4 quad_move(Word4 v) {
+    Word4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = __builtin_amdgcn_mov_dpp(static_cast<int>(v[i]), ctrl, 0xF, 0xF, true);
+    return r;
+}
+__device__ __forceinline__ void share_entry(__amdgpu_buffer_rsrc_t buf, unsigned int off, const Real (&p)[8]) {
+    const int l = threadIdx.x & 3;
+    Word4 a[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = __builtin_bit_cast(Word4, Pair16{p[2 * i], p[2 * i + 1]});
+    // a 4 x 4 transposition: with the lane beside (quad_perm 1 0 3 2), then with the lane two over (2 3 0 1)
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+        const Word4 y = quad_move<0xB1>(l & 1 ? a[i] : a[i + 1]);
+        a[i] = l & 1 ? y : a[i];
+        a[i + 1] = l & 1 ? a[i + 1] : y;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const Word4 y = quad_move<0x4E>(l & 2 ? a[i] : a[i + 2]);
+        a[i] = l & 2 ? y : a[i];
+        a[i + 2] = l & 2 ? a[i + 2] : y;
+    }
+    auto put = [&](Word4 v, int first) {   // piece l of the entry of the quad's lane whose offset is `first`
+        if (first != static_cast<int>(kNoEntry))
+            __builtin_amdgcn_raw_buffer_store_b128(v, buf, static_cast<unsigned int>(first) + 16 * l, 0, kAgentScope);
+    };
+    put(a[0], __builtin_amdgcn_mov_dpp(static_cast<int>(off), 0x00, 0xF, 0xF, true));
+    put(a[1], __builtin_amdgcn_mov_dpp(static_cast<int>(off), 0x55, 0xF, 0xF, true));
+    put(a[2], __builtin_amdgcn_mov_dpp(static_cast<int>(off), 0xAA, 0xF, 0xF, true));
+    put(a[3], __builtin_amdgcn_mov_dpp(static_cast<int>(off), 0xFF, 0xF, 0xF, true));
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t shared_buffer(const Real* p, size_t doubles) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<Real*>(p), 0, static_cast<int>(doubles * sizeof(Real)), 0x00020000);
+}
 
 // Grid barrier of the G workgroups of a run.  `target` counts this workgroup's barriers; the shared counter only
 // grows, so barrier n completes when it reaches n G.  Returns false (and sets the run's error flag) when the
 // others do not arrive in time, or when another workgroup has already given up.
-// One release fence before the arrival and one acquire fence after the wait, with the counter itself relaxed
-// (fence-to-fence synchronisation through the counter's release sequence): on this GPU an agent-scope release
-// writes back the die's whole L2 and an acquire invalidates it, operations every other kernel on the die waits
-// behind, so the barrier issues them once and none per poll.
+// Every wave waits until its own stores are complete (a workgroup's barrier does not wait for that, and the release fence
+// of one wave waits for that wave's stores alone); then one release fence before the arrival and one acquire fence after
+// the wait, with the counter itself relaxed (fence-to-fence synchronisation through the counter's release sequence).  An
+// agent-scope release writes back the die's whole L2 and an acquire invalidates it, operations every other kernel on the
+// die waits behind, so the barrier issues one of each and none per poll.
 __device__ __forceinline__ bool grid_sync(unsigned int* __restrict__ ctr, unsigned int* __restrict__ err, int G,
                                           unsigned int& target, int* s_ok) {
-    wait_stores();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     target += 1;
     if (threadIdx.x == 0) {
         int ok = 1;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");   // this workgroup's writes before the arrival
-        // A second write-back after the first is done.  With one, and the workgroups of other launches writing back the
-        // same die's L2 at the same time, lines made dirty just before the barrier could still be in this L2 when others
-        // read them: 16 of 20 sequences of 16 steps with three in flight read old list entries.  With two none did in 20,
-        // nor with entries stored through to memory (391 us a slice against 353).  A write-back that runs when a request
-        // arrives may have passed those lines; one that starts after the first has ended has not.
-        asm volatile("buffer_wbl2 sc1\n\ts_waitcnt vmcnt(0)" ::: "memory");
         __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const unsigned int want = target * static_cast<unsigned int>(G);
         const unsigned long long t0 = wall_clock64();
@@ -148,8 +245,8 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
 
     const int N = A.grid.N, M = N + 1;
     const Real R = A.grid.R;
-    Real* __restrict__ ws = A.ws;
-    auto WS = [&](int arr) -> Real* { return ws + static_cast<size_t>(arr) * M; };
+    const Real* ws = A.ws;   // written through share()
+    auto WS = [&](int arr) -> const Real* { return ws + static_cast<size_t>(arr) * M; };
     const int K = A.nslices;
     const int kb = A.k_begin, ke = A.k_end > 0 ? A.k_end : K;
     const Real dxi = A.dxi;
@@ -168,15 +265,16 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
 
     // the run's multi-workgroup workspace
     const MwsLayout mw(M, N, NP, G, M1);
-    Real* __restrict__ mws = A.mws;
+    Real* mws = A.mws;
     unsigned int* bar = reinterpret_cast<unsigned int*>(mws);
     unsigned int* err = bar + 2;
-    Real* g_bw0 = mws + 8;
-    int* g_cnt = reinterpret_cast<int*>(mws + mw.cnt);
-    Real* __restrict__ g_list = mws + mw.lists;
-    const size_t lstride = 2 * static_cast<size_t>(NP > 1 ? NP : 1);
+    const Real* g_bw0 = mws + 8;
+    const int* g_cnt = reinterpret_cast<const int*>(mws + mw.cnt);
+    const Real* g_list = mws + mw.lists;
+    const __amdgpu_buffer_rsrc_t list_buf = shared_buffer(g_list, mw.bpalt - mw.lists);
+    const __amdgpu_buffer_rsrc_t fac_buf = shared_buffer(WS(W_FAC0), 8 * static_cast<size_t>(M));
     Real* __restrict__ g_gath = mws + mw.gath;
-    Real* bpbuf[2] = {WS(W_BPR1), mws + mw.bpalt};   // Picard iterates: W_BPR1.. of ws, then the second buffer
+    const Real* bpbuf[2] = {WS(W_BPR1), mws + mw.bpalt};   // Picard iterates: W_BPR1.. of ws, then the second buffer
     unsigned int nbar = 0;
 
     // LDS
@@ -191,7 +289,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
     int* s_goff = reinterpret_cast<int*>(smem + plan.goff);
     unsigned short* s_sidx = reinterpret_cast<unsigned short*>(smem + plan.sidx);
     int* s_misc = reinterpret_cast<int*>(smem + plan.misc);   // [0] barrier verdict [1] live [2] last cell count
-    int* s_comps = s_misc + 8;                                 // the deposit arrays of this run, in pass order
+    int* s_code = s_misc + 8;                                  // entry_code of every slot
     int& s_ok = s_misc[0];
     int& s_live = s_misc[1];
     Real* B = reinterpret_cast<Real*>(smem + plan.region);
@@ -207,27 +305,8 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
     }
     if (kb == 0)   // B+ := 0 at the head (Simulation.cpp:705-708); every workgroup its share of the nodes
         for (int j = grp * mBS + tid; j < M; j += gthreads)
-            for (int a = 0; a < (M1 ? 6 : 2); ++a) WS(W_BPR1 + a)[j] = Real(0);
-    // deposit arrays of this run in a fixed order
-    int ncomp = 0;
-    {
-        auto put = [&](int c) {
-            if (tid == 0) s_comps[ncomp] = c;
-            ++ncomp;
-        };
-        put(W_CHI0); put(W_RHOT0); put(W_DRHO0); put(W_JZ0);
-        if (has_neg) put(W_NE0);
-        if (has_pos) put(W_NI0);
-        put(W_JPR1); put(W_JPI1);
-        if (M1) {
-            put(W_CHI1R); put(W_CHI1I); put(W_RHOT1R); put(W_RHOT1I); put(W_DRHO1R); put(W_DRHO1I);
-            put(W_JZ1R); put(W_JZ1I);
-            if (has_neg) { put(W_NE1R); put(W_NE1I); }
-            if (has_pos) { put(W_NI1R); put(W_NI1I); }
-            put(W_JPR0); put(W_JPI0); put(W_JPR2); put(W_JPI2);
-        }
-    }
-    const int nS = M1 ? 6 : 2;
+            for (int a = 0; a < (M1 ? 6 : 2); ++a) share(WS(W_BPR1 + a) + j, Real(0));
+    for (int i = tid; i < SL::ENTRY; i += mBS) s_code[i] = entry_code(i, has_neg, has_pos);
     const Real dmin = A.delta_min, qsamax = A.max_qsa;
     const int ord = A.ab_order;
     const int niter = M1 ? A.picard : 1;
@@ -326,7 +405,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                 run_ += v;
             }
             s_cs[c + 1] = run_;
-            g_cnt[static_cast<size_t>(grp) * N + c] = run_;
+            share(g_cnt + static_cast<size_t>(grp) * N + c, run_);
         }
         __syncthreads();
         const int Lloc = s_live;
@@ -371,10 +450,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
         // The two contributions of every owned particle get their positions in the run's node lists: node n holds cell
         // n-1 (right entries) and cell n (left entries), merged in particle-index order, and this workgroup's entries are
         // one run of it after those of the earlier workgroups.  Of the position only that among the workgroup's own
-        // entries is kept, in 16 bits a side; the offset of the run follows from the cell.  The entries go to memory as
-        // they are formed, all components of a particle in turn: a store of a wave takes a line per lane, but nothing
-        // waits for it.  Gathered in LDS in list order first and copied out coalesced they take longer (m = 1, 32768
-        // particles over 8 workgroups 444 us a slice against 353; 8192 over 4 136.6 against 130).
+        // entries is kept, in 16 bits a side; the offset of the run follows from the cell.
 #pragma unroll
         for (int pp = 0; pp < PT; ++pp) {
             const int j = cj[pp];
@@ -424,37 +500,32 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
 #pragma unroll
                 for (int u = 0; u < PB; ++u) {
                     const int pp = p0 + u;
-                    const int j = cj[pp];
-                    if (j < 0) continue;
+                    const bool live = cj[pp] >= 0;
+                    const int j = max(cj[pp], 0);   // lanes without a particle take part in the exchanges
                     const Real PX = PXb[u], PY = PYb[u], D = Db[u], wi = wb[u];
                     const bool s1 = own0 + slot_of(pp) >= np0;
                     const Real q = s1 ? q1 : q0, qm = s1 ? qm1 : qm0;
-                    const int gl = (cpos[pp] & 0xffff) + shift(j), gr = (cpos[pp] >> 16) + shift(j + 1);
-                    const Real ih = s_ih[j], iv0 = s_iv[j], iv1 = s_iv[j + 1];
+                    const Real ih = s_ih[j];
                     const Real pz = cgam[pp] - D;
-                    Real* __restrict__ L = g_list;
-                    auto pass = [&](auto... cst) {
-                        ((L[gl] = dep_value(decltype(cst)::value, 0, j, ct[pp], cc[pp], cs[pp], cir[pp], cinvd[pp], cgam[pp], PX,
-                                            PY, pz, wi, q, qm, iv0, ih),
-                          L[gr] = dep_value(decltype(cst)::value, 1, j, ct[pp], cc[pp], cs[pp], cir[pp], cinvd[pp], cgam[pp], PX,
-                                            PY, pz, wi, q, qm, iv1, ih),
-                          L += lstride),
-                         ...);
-                    };
-                    pass(IC<W_CHI0>{}, IC<W_RHOT0>{});
-                    pass(IC<W_DRHO0>{}, IC<W_JZ0>{});
-                    if (has_neg) pass(IC<W_NE0>{});
-                    if (has_pos) pass(IC<W_NI0>{});
-                    pass(IC<W_JPR1>{}, IC<W_JPI1>{});
-                    if constexpr (M1) {
-                        pass(IC<W_CHI1R>{}, IC<W_CHI1I>{});
-                        pass(IC<W_RHOT1R>{}, IC<W_RHOT1I>{});
-                        pass(IC<W_DRHO1R>{}, IC<W_DRHO1I>{});
-                        pass(IC<W_JZ1R>{}, IC<W_JZ1I>{});
-                        if (has_neg) pass(IC<W_NE1R>{}, IC<W_NE1I>{});
-                        if (has_pos) pass(IC<W_NI1R>{}, IC<W_NI1I>{});
-                        pass(IC<W_JPR0>{}, IC<W_JPI0>{});
-                        pass(IC<W_JPR2>{}, IC<W_JPI2>{});
+#pragma unroll
+                    for (int side = 0; side < 2; ++side) {
+                        const int at = (side == 0 ? (cpos[pp] & 0xffff) : (cpos[pp] >> 16)) + shift(j + side);
+                        const unsigned int off = static_cast<unsigned int>(at) * (SL::ENTRY * 8);
+                        const Real iv = s_iv[j + side];
+                        auto pass = [&](auto first) {   // eight of the entry's arrays, from entry_comp(first)
+                            constexpr int S = decltype(first)::value;
+                            Real v[8];
+                            for_each_batch<8>([&](auto i) {
+                                v[i] = dep_value(entry_comp(S + i), side, j, ct[pp], cc[pp], cs[pp], cir[pp], cinvd[pp], cgam[pp],
+                                                 PX, PY, pz, wi, q, qm, iv, ih);
+                            });
+                            share_entry(list_buf, live ? off + S * 8 : kNoEntry, v);
+                        };
+                        pass(IC<0>{});
+                        if constexpr (M1) {
+                            pass(IC<8>{});
+                            pass(IC<16>{});
+                        }
                     }
                 }
             }
@@ -466,51 +537,45 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
             const Real* __restrict__ bs = A.bsrc;
             const Real* __restrict__ bg = A.bg;
             const bool ngp = A.ngp != 0;
-            auto bb = [&](int kk, int j, int comp) { return bs[(static_cast<size_t>(kk) * M + j) * ncb + comp]; };
-            auto dxi_b = [&](int j, int comp) {   // combine_sources' xi derivative of the beam source
-                if (ngp) {
-                    const Real prev = (k > 0) ? bb(k - 1, j, comp) : Real(0);
-                    return (bb(k, j, comp) - prev) * idxi;
-                }
-                if (K == 1) return Real(0);
-                if (k == 0) return (bb(1, j, comp) - bb(0, j, comp)) * idxi;
-                if (k == K - 1) return (bb(K - 1, j, comp) - bb(K - 2, j, comp)) * idxi;
-                return Real(0.5) * (bb(k + 1, j, comp) - bb(k - 1, j, comp)) * idxi;
-            };
-            for (int item = gtid; item < ncomp * M; item += gthreads) {
-                const int ci = item / M, n = item - ci * M;
+            // combine_sources' xi derivative of a beam source: half (row hi - row lo) / dxi, row -1 zero
+            const int hi = ngp || k == K - 1 ? k : k + 1, lo = ngp || k > 0 ? k - 1 : 0;
+            const Real half = ngp || k == 0 || k == K - 1 ? Real(1) : Real(0.5);
+            const bool flat = !ngp && K == 1;
+            // a wave sums the lists of eight nodes: eight lanes read 64 bytes of an entry side by side, a lane the same double
+            // of each such part, and the sums of eight nodes are stored side by side.  Bound by the trips to memory: 29 us
+            // a slice (m = 1, 1025 nodes, 64 entries a node, 8 workgroups), 42 us with the sources read after the sums,
+            // 9 and 18 us with 513 nodes and 16 entries.  11 entries in flight beside eight particles per thread: 12
+            // spill.
+            constexpr int P = SL::ENTRY / 8;
+            for (int tile = grp * mNW + w; tile < (M + 7) / 8; tile += G * mNW) {
+                const int n = 8 * tile + (lane >> 3);
+                if (n >= M) continue;
                 const int e0 = s_gcs[n] + s_gcs[n + 1], e1 = s_gcs[n + 1] + s_gcs[n + 2];
-                const Real acc = sum_list_pairs(g_list + static_cast<size_t>(ci) * lstride, e0, e1);
-                const int comp = s_comps[ci];
-                Real* Dn = Dg + static_cast<size_t>(n) * ncd;
-                // the node sum combined with the background and the beam sources (Simulation.cpp:408-457)
-                switch (comp) {
-                    case W_RHOT0: WS(comp)[n] = acc + (bg[n] + bb(k, n, B_RT0)); break;
-                    case W_DRHO0: WS(comp)[n] = acc + dxi_b(n, B_RT0); break;
-                    case W_JZ0: WS(comp)[n] = acc + bb(k, n, B_JZ0); break;
-                    case W_JPR1: WS(comp)[n] = acc + bb(k, n, B_JP1R); break;
-                    case W_JPI1: WS(comp)[n] = acc + bb(k, n, B_JP1I); break;
-                    case W_RHOT1R: WS(comp)[n] = acc + (bg[M + n] + bb(k, n, B_RT1R)); break;
-                    case W_RHOT1I: WS(comp)[n] = acc + (bg[2 * M + n] + bb(k, n, B_RT1I)); break;
-                    case W_DRHO1R: WS(comp)[n] = acc + dxi_b(n, B_RT1R); break;
-                    case W_DRHO1I: WS(comp)[n] = acc + dxi_b(n, B_RT1I); break;
-                    case W_JZ1R: WS(comp)[n] = acc + bb(k, n, B_JZ1R); break;
-                    case W_JZ1I: WS(comp)[n] = acc + bb(k, n, B_JZ1I); break;
-                    case W_JPR0: WS(comp)[n] = acc + bb(k, n, B_JP0R); break;
-                    case W_JPI0: WS(comp)[n] = acc + bb(k, n, B_JP0I); break;
-                    case W_JPR2: WS(comp)[n] = acc + bb(k, n, B_JP2R); break;
-                    case W_JPI2: WS(comp)[n] = acc + bb(k, n, B_JP2I); break;
-                    case W_NE0: Dn[D_NE0] = acc; break;
-                    case W_NE1R: Dn[D_NE1R] = acc; break;
-                    case W_NE1I: Dn[D_NE1I] = acc; break;
-                    case W_NI1R: Dn[D_NI1R] = acc; break;
-                    case W_NI1I: Dn[D_NI1I] = acc; break;
-                    case W_NI0: {   // combine_sources adds the positive background (Simulation.cpp:441)
-                        const Real bgr0 = bg[3 * M + n];
-                        Dn[D_NI0] = bgr0 > Real(0) ? acc + bgr0 : acc;
-                        break;
-                    }
-                    default: WS(comp)[n] = acc;   // chi
+                // the sources are on their way while the lists are summed
+                int code[P];
+                Real u[P], v[P], sums[P];
+#pragma unroll
+                for (int part = 0; part < P; ++part) {
+                    code[part] = s_code[8 * part + (lane & 7)];
+                    const int c = max(code[part], 0), kind = c & 15, beam = c >> 12 & 255;
+                    const bool from_bg = kind == kKindBackground || kind == kKindIons, dxi_b = kind == kKindDxi;
+                    u[part] = *(from_bg ? bg + (c >> 20) * M + n
+                                        : bs + (static_cast<size_t>(dxi_b ? hi : k) * M + n) * ncb + beam);
+                    v[part] = bs[(static_cast<size_t>(dxi_b ? max(lo, 0) : k) * M + n) * ncb + beam];
+                }
+                sum_rows<SL::ENTRY, P, (P == 1 || PT <= 4 ? 16 : 11)>(g_list + (lane & 7), e0, e1, sums);
+#pragma unroll
+                for (int part = 0; part < P; ++part) {
+                    const int kind = code[part] & 15, dst = code[part] >> 4 & 255;
+                    Real acc = sums[part];
+                    if (code[part] < 0) continue;
+                    if (kind == kKindBackground) acc = acc + (u[part] + v[part]);
+                    if (kind == kKindBeam) acc = acc + u[part];
+                    if (kind == kKindDxi)
+                        acc = acc + (flat ? Real(0) : half * (u[part] - (lo < 0 ? Real(0) : v[part])) * idxi);
+                    if (kind == kKindIons && u[part] > Real(0)) acc = acc + u[part];   // Simulation.cpp:441
+                    if (kind >= kKindDiag) Dg[static_cast<size_t>(n) * ncd + dst] = acc;
+                    else share(WS(dst) + n, acc);
                 }
             }
             // densities of absent species are zero, plus the positive background for n_i
@@ -577,16 +642,16 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                 // results: psi over its right-hand side in ws, E_z and B_z to their arrays
                 for (int j = tid; j < M; j += mBS) {
                     if (l0) {
-                        WS(W_RHOT0)[j] = BA(3)[j];
-                        WS(W_EZ0)[j] = BA(4)[j];
-                        WS(W_BZ0)[j] = BA(5)[j];
+                        share(WS(W_RHOT0) + j, BA(3)[j]);
+                        share(WS(W_EZ0) + j, BA(4)[j]);
+                        share(WS(W_BZ0) + j, BA(5)[j]);
                     } else {
-                        WS(W_RHOT1R)[j] = BA(3)[j];
-                        WS(W_RHOT1I)[j] = BA(4)[j];
-                        WS(W_EZ1R)[j] = BA(5)[j];
-                        WS(W_EZ1I)[j] = BA(6)[j];
-                        WS(W_BZ1R)[j] = BA(7)[j];
-                        WS(W_BZ1I)[j] = BA(8)[j];
+                        share(WS(W_RHOT1R) + j, BA(3)[j]);
+                        share(WS(W_RHOT1I) + j, BA(4)[j]);
+                        share(WS(W_EZ1R) + j, BA(5)[j]);
+                        share(WS(W_EZ1I) + j, BA(6)[j]);
+                        share(WS(W_BZ1R) + j, BA(7)[j]);
+                        share(WS(W_BZ1I) + j, BA(8)[j]);
                     }
                 }
                 __syncthreads();
@@ -608,8 +673,12 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     const int op = f == 0 ? OP_L1D : f == 1 ? OP_L1F : f == 2 ? OP_L0 : OP_L2D;
                     const Real aN = A.op_a[op][N], bN = A.op_b[op][N];
                     const bool dir0 = op != OP_L0, dirN = op != OP_L1F;
-                    g_bw0[f] = thomas_factor_wave<kRows>(BA(base), BA(base + 1), BA(base + 2), BA(3), aN, bN, dir0, dirN,
-                                                  WS(W_FAC0 + 2 * f), WS(W_FAC0 + 2 * f + 1), M);
+                    // m and c' of a row side by side, operator after operator
+                    share(g_bw0 + f,
+                          thomas_factor_wave<kRows>(BA(base), BA(base + 1), BA(base + 2), BA(3), aN, bN, dir0, dirN, M,
+                                                    [&](int i, Real m, Real cp) {
+                                                        share_pair(fac_buf, (static_cast<unsigned int>(f) * M + i) * 16, m, cp);
+                                                    }));
                 }
                 __syncthreads();
             }
@@ -649,7 +718,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                 Dj[D_PSI0] = psi0[j];
                 Fj[F_EZ0] = BA(SL::EZ)[j];
                 Fj[F_BZ0] = BA(SL::BZ)[j];
-                for (int a = 0; a < (M1 ? 6 : 2); ++a) WS(W_WPR1 + a)[j] = BA(SL::W + a)[j];
+                for (int a = 0; a < (M1 ? 6 : 2); ++a) share(WS(W_WPR1 + a) + j, BA(SL::W + a)[j]);
                 if (M1) {
                     Dj[D_PSI1R] = psr[j]; Dj[D_PSI1I] = psi_[j];
                     Fj[F_EZ1R] = BA(SL::EZ + 1)[j]; Fj[F_EZ1I] = BA(SL::EZ + 2)[j];
@@ -666,8 +735,8 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
 #pragma unroll
                 for (int u = 0; u < PB; ++u) {
                     const int pp = p0 + u;
-                    const int j = cj[pp];
-                    if (j < 0) continue;
+                    const bool live = cj[pp] >= 0;
+                    const int j = max(cj[pp], 0);
                     const Real PX = PXb[u], PY = PYb[u], wi = wb[u];
                     const bool s1 = own0 + slot_of(pp) >= np0;
                     const Real qq = s1 ? q1 : q0, qm = s1 ? qm1 : qm0;
@@ -685,7 +754,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                                                 M1 ? lin(BA(SL::EZ + 2), j, t) : Real(0), c, sn, M1);
                     const Real Bz = eval_scalar(lin(BA(SL::BZ), j, t), M1 ? lin(BA(SL::BZ + 1), j, t) : Real(0),
                                                 M1 ? lin(BA(SL::BZ + 2), j, t) : Real(0), c, sn, M1);
-                    {
+                    if (live) {
                         Real* gt = g_gath + own0 + slot_of(pp);
                         gt[0] = Wx;
                         gt[static_cast<size_t>(NP)] = Wy;
@@ -702,16 +771,18 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     const Real ur = c * ux + sn * uy, uth = c * uy - sn * ux;
                     const Real wq = wi * qq;
                     const Real ih = s_ih[j];
-                    Real* __restrict__ L = g_list;
-                    auto s_pass = [&](auto cst) {   // the real and imaginary components of one mode
-                        constexpr int mode = decltype(cst)::value;
-                        const Real ck = mode == 1 ? c : (mode == 0 ? Real(1) : c * c - sn * sn);
-                        const Real sk = mode == 1 ? sn : (mode == 0 ? Real(0) : Real(2) * c * sn);
 #pragma unroll
-                        for (int side = 0; side < 2; ++side) {
-                            const Real iv = s_iv[j + side] * wq;
-                            const Real W = side == 0 ? Real(1) - t : t;
-                            const Real dW = side == 0 ? -ih : ih;
+                    for (int side = 0; side < 2; ++side) {
+                        const int at = (side == 0 ? (cpos[pp] & 0xffff) : (cpos[pp] >> 16)) + shift(j + side);
+                        const unsigned int off = static_cast<unsigned int>(at) * (SL::SENTRY * 8);
+                        const Real iv = s_iv[j + side] * wq;
+                        const Real W = side == 0 ? Real(1) - t : t;
+                        const Real dW = side == 0 ? -ih : ih;
+                        Real v[8] = {};
+                        auto s_pass = [&](auto cst, int slot) {   // the real and imaginary components of one mode
+                            constexpr int mode = decltype(cst)::value;
+                            const Real ck = mode == 1 ? c : (mode == 0 ? Real(1) : c * c - sn * sn);
+                            const Real sk = mode == 1 ? sn : (mode == 0 ? Real(0) : Real(2) * c * sn);
                             Real Ar = ax * W + ux * ur * dW;
                             Real Ai = ay * W + uy * ur * dW;
                             if (mode != 0) {
@@ -720,25 +791,33 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                                 Ar += f2 * uy;
                                 Ai -= f2 * ux;
                             }
-                            const int at = (side == 0 ? (cpos[pp] & 0xffff) : (cpos[pp] >> 16)) + shift(j + side);
-                            L[at] = iv * (Ar * ck + Ai * sk);
-                            L[lstride + at] = iv * (Ai * ck - Ar * sk);
+                            v[slot] = iv * (Ar * ck + Ai * sk);
+                            v[slot + 1] = iv * (Ai * ck - Ar * sk);
+                        };
+                        s_pass(IC<1>{}, 0);
+                        if constexpr (M1) {
+                            s_pass(IC<0>{}, 2);
+                            s_pass(IC<2>{}, 4);
+                            share_entry(list_buf, live ? off : kNoEntry, v);
+                        } else if (live) {
+                            share_pair(list_buf, off, v[0], v[1]);
                         }
-                        L += 2 * lstride;
-                    };
-                    s_pass(IC<1>{});
-                    if constexpr (M1) {
-                        s_pass(IC<0>{});
-                        s_pass(IC<2>{});
                     }
                 }
             }
         }
         if (!(alive = grid_sync(bar, err, G, nbar, &s_ok))) break;
-        for (int item = gtid; item < nS * M; item += gthreads) {
-            const int sc = item / M, n = item - sc * M;
-            const int e0 = s_gcs[n] + s_gcs[n + 1], e1 = s_gcs[n + 1] + s_gcs[n + 2];
-            WS(W_SR1 + sc)[n] = sum_list_pairs(g_list + static_cast<size_t>(sc) * lstride, e0, e1);
+        {
+            constexpr int nodes = 64 / SL::NS;   // of a wave
+            const int tiles = (M + nodes - 1) / nodes;
+            for (int tile = grp * mNW + w; tile < tiles; tile += G * mNW) {
+                const int u = lane / SL::NS, sc = lane - u * SL::NS, n = tile * nodes + u;
+                if (u >= nodes || n >= M) continue;
+                const int e0 = s_gcs[n] + s_gcs[n + 1], e1 = s_gcs[n + 1] + s_gcs[n + 2];
+                Real acc[1];
+                sum_rows<SL::SENTRY, 1, 16>(g_list + sc, e0, e1, acc);
+                share(WS(W_SR1 + sc) + n, acc[0]);
+            }
         }
         if (!(alive = grid_sync(bar, err, G, nbar, &s_ok))) break;
 
@@ -750,7 +829,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
             const Real fcw = A.flux_coef * WS(W_JZ0)[N];
             for (int it = 0; it < niter; ++it) {
                 const Real* bp = bpbuf[it & 1];
-                Real* bn = bpbuf[(it + 1) & 1];
+                const Real* bn = bpbuf[(it + 1) & 1];
                 auto BP = [&](int f, int j) { return bp[static_cast<size_t>(f) * M + j]; };
                 for (int job = grp; job < njob; job += G) {
                     // slots: 0 a (first system), 1 a (second), 2,3 factors of the first, 4,5 of the second,
@@ -768,32 +847,33 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                             gr = BA(8)[j];
                             gi = BA(9)[j];
                         } else {
-                        BA(0)[j] = A.op_a[opa][j];
-                        BA(1)[j] = A.op_a[opb][j];
-                        BA(2)[j] = WS(W_FAC0 + 2 * fa)[j]; BA(3)[j] = WS(W_FAC0 + 2 * fa + 1)[j];
-                        BA(4)[j] = WS(W_FAC0 + 2 * fb)[j]; BA(5)[j] = WS(W_FAC0 + 2 * fb + 1)[j];
-                        // gz: ((d_x + i d_y) J_z)_k + S_k, and the chi_1 coupling with the previous iterate
-                        if (job == 0) {
-                            const Real t1 = stn.grad(WS(W_JZ0), j);
-                            gr = t1 + WS(W_SR1)[j];
-                            gi = WS(W_SI1)[j];
-                        } else {
-                            const Real* fr = WS(W_JZ1R);
-                            const Real* fi = WS(W_JZ1I);
-                            const Real t2 = stn.grad_odd(fr, j), t3 = stn.over_r(fr, j);
-                            const Real t4 = stn.grad_odd(fi, j), rh = stn.over_r(fi, j);
-                            if (job == 1) {
-                                gr = (t2 + t3) + WS(W_SR0)[j];
-                                gi = -(t4 + rh) + WS(W_SI0)[j];
+                            BA(0)[j] = A.op_a[opa][j];
+                            BA(1)[j] = A.op_a[opb][j];
+                            const Real *fca = WS(W_FAC0 + 2 * fa) + 2 * j, *fcb = WS(W_FAC0 + 2 * fb) + 2 * j;
+                            BA(2)[j] = fca[0]; BA(3)[j] = fca[1];
+                            BA(4)[j] = fcb[0]; BA(5)[j] = fcb[1];
+                            // gz: ((d_x + i d_y) J_z)_k + S_k, and the chi_1 coupling with the previous iterate
+                            if (job == 0) {
+                                const Real t1 = stn.grad(WS(W_JZ0), j);
+                                gr = t1 + WS(W_SR1)[j];
+                                gi = WS(W_SI1)[j];
                             } else {
-                                gr = (t2 - t3) + WS(W_SR2)[j];
-                                gi = (t4 - rh) + WS(W_SI2)[j];
+                                const Real* fr = WS(W_JZ1R);
+                                const Real* fi = WS(W_JZ1I);
+                                const Real t2 = stn.grad_odd(fr, j), t3 = stn.over_r(fr, j);
+                                const Real t4 = stn.grad_odd(fi, j), rh = stn.over_r(fi, j);
+                                if (job == 1) {
+                                    gr = (t2 + t3) + WS(W_SR0)[j];
+                                    gi = -(t4 + rh) + WS(W_SI0)[j];
+                                } else {
+                                    gr = (t2 - t3) + WS(W_SR2)[j];
+                                    gi = (t4 - rh) + WS(W_SI2)[j];
+                                }
                             }
-                        }
-                        if (M1) {
-                            BA(8)[j] = gr;
-                            BA(9)[j] = gi;
-                        }
+                            if (M1) {
+                                BA(8)[j] = gr;
+                                BA(9)[j] = gi;
+                            }
                         }
                         Real rr = -gi, ri = gr;
                         if (M1) {
@@ -822,8 +902,8 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     }
                     __syncthreads();
                     for (int j = tid; j < M; j += mBS) {
-                        bn[static_cast<size_t>(sys0) * M + j] = BA(6)[j];
-                        bn[static_cast<size_t>(sys0 + 1) * M + j] = BA(7)[j];
+                        share(bn + static_cast<size_t>(sys0) * M + j, BA(6)[j]);
+                        share(bn + static_cast<size_t>(sys0 + 1) * M + j, BA(7)[j]);
                     }
                     __syncthreads();
                 }
@@ -854,7 +934,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
                     Fj[F_BP0R] = b0r; Fj[F_BP0I] = b0i; Fj[F_BP2R] = b2r; Fj[F_BP2I] = b2i;
                 }
                 if (niter & 1)   // the warm start of the next slice goes back to ws
-                    for (int f = 0; f < (M1 ? 6 : 2); ++f) WS(W_BPR1 + f)[j] = BF(f, j);
+                    for (int f = 0; f < (M1 ? 6 : 2); ++f) share(WS(W_BPR1 + f) + j, BF(f, j));
             }
             if (k < K - 1) {
                 // ---- Adams-Bashforth push (PlasmaSpecies::push, src/PlasmaSpecies.cpp:600-667); B+ staged in LDS

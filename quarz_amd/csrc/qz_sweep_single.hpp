@@ -652,8 +652,10 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
             const int op = f == 0 ? OP_L1D : f == 1 ? OP_L1F : f == 2 ? OP_L0 : OP_L2D;
             const Real aN = A.op_a[op][N], bN = A.op_b[op][N];
             const bool dir0 = op != OP_L0, dirN = op != OP_L1F;
-            s_bw0[f] = thomas_factor_wave<kRows>(a, b, c, BA(LY::CHI0), aN, bN, dir0, dirN, WS(W_FAC0 + 2 * f),
-                                          WS(W_FAC0 + 2 * f + 1), M);
+            Real* __restrict__ fm = WS(W_FAC0 + 2 * f);
+            Real* __restrict__ fc = WS(W_FAC0 + 2 * f + 1);
+            s_bw0[f] = thomas_factor_wave<kRows>(a, b, c, BA(LY::CHI0), aN, bN, dir0, dirN, M,
+                                                 [&](int i, Real m, Real cp) { fm[i] = m; fc[i] = cp; });
         }
         __syncthreads();
         QZ_PHASE(6);
