@@ -47,13 +47,13 @@ namespace qz {
 // the backward sweep reads.
 typedef double Pair8 __attribute__((ext_vector_type(2), aligned(8)));   // two doubles at any double's address
 
-// Systems stored row after row (kRows: es = 1), and few systems of any layout: a DPP row of 16 lanes per system, 8 rows
-// per lane in registers (qz_chain.hpp), so that a lane reads whole cache lines and a sixteenth of the systems that one
-// thread each would need fills the chip.  The next block of rows is loaded while one is run.  The reciprocal is
+// Long systems stored row after row (kRows: es = 1), and few systems of any layout: a DPP row of 16 lanes per system, 8
+// rows per lane in registers (qz_chain.hpp), so that a lane reads whole cache lines and a sixteenth of the systems that
+// one thread each would need fills the chip.  The next block of rows is loaded while one is run.  The reciprocal is
 // chain_recip, checked against the division after each block.  Bound by the chain up to 4096 systems, then by its
 // repeated steps.
-// Row after row: 4096 systems of 513 rows 42 us (2.0 TB/s), where one thread per system, a row at a time, took 405 us;
-// 4 systems of 65 rows 7 us (22 us).
+// Row after row: 4096 systems of 513 rows 41 us (2.1 TB/s), where one thread per system, a row at a time, took 412 us;
+// 64 systems of 65 rows 6 us (31 us).
 template <bool kRows>
 __global__ void __launch_bounds__(64) thomas_lanes_kernel(const Real* a, const Real* b, const Real* c, const Real* d,
                                                           Real* x, Real* cpw, int M, int batch, long long ss,
@@ -196,13 +196,12 @@ __global__ void __launch_bounds__(64) thomas_lanes_kernel(const Real* a, const R
     }
 }
 
-// Any strides: one thread per system, eight rows loaded ahead of the eight being run; c' element-major.
+// Any strides: one thread per system, U rows loaded ahead of the U being run; c' element-major.
 // Element-major, 513 rows: 32768 systems 218 us (3.1 TB/s), 576 us without the loads ahead.
-constexpr int kThomasAhead = 8;
+template <int U>
 __global__ void __launch_bounds__(64) thomas_batched_kernel(const Real* a, const Real* b, const Real* c, const Real* d,
                                                             Real* x, Real* cpw, int M, int batch, long long ss,
                                                             long long es) {
-    constexpr int U = kThomasAhead;
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= batch) return;
     const long long o = static_cast<long long>(s) * ss;
@@ -260,10 +259,17 @@ __global__ void __launch_bounds__(64) thomas_batched_kernel(const Real* a, const
 }
 }  // namespace qz
 
-// Systems up to which systems that are not stored row after row take a DPP row per system, whose lanes then read 8
-// bytes of every line: 513 rows, 2048 systems 57 us against 100 us for a thread per system, 4096 86 against 98, 8192
-// 166 against 102.  Systems stored row after row always do: 65536 systems 0.58 ms against 1.9 ms.
+// Up to kThomasLanesMax systems each takes a DPP row, in any layout (element-major, 513 rows: 2048 systems 57 us against
+// 100 us for a thread per system, 4096 86 against 98, 8192 166 against 102).  Of more, those stored row after row with
+// more than kThomasThreadRows rows do: a wave runs whole blocks of 8 rows per lane and checks them, whatever a system
+// has, and a thread per system is faster while its rows lie in a few cache lines.  Row after row, DPP row against thread:
+//   10^6 systems of   2 rows 503 us / 19,   9 rows 682 / 193,   17 rows 751 / 693,   18 rows 759 / 896,   33 rows 863 / 1651
+//   8192 systems of   2 rows 6.2 us / 5.4,  9 rows 7.1 / 5.8,   17 rows 7.5 / 6.3,   18 rows 7.7 / 7.0,   33 rows 8.9 / 9.8
 constexpr int kThomasLanesMax = 4096;
+constexpr int kThomasThreadRows = 17;
+// Rows a thread loads ahead: two for systems that have no more after the first, where eight would be loads of the last
+// row (2 rows, 4 x 10^6 systems row after row: 89 us, 146 us with eight).
+constexpr int kThomasTinyRows = 3;
 
 extern "C" size_t qz_tridiag_workspace_doubles(int M, int batch) {
     return (M < 1 || batch < 1) ? 0 : static_cast<size_t>(M) * static_cast<size_t>(batch);
@@ -285,15 +291,15 @@ extern "C" int qz_tridiag_thomas_batched(const double* a, const double* b, const
             if ((si * sys_stride) % elem_stride == 0)
                 return qz_fail(QZ_EINVAL, "qz_tridiag_thomas_batched: strides make two systems overlap");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (elem_stride == 1 || batch <= kThomasLanesMax) {
+    if (batch <= kThomasLanesMax || (elem_stride == 1 && M > kThomasThreadRows)) {
         hipLaunchKernelGGL(elem_stride == 1 ? qz::thomas_lanes_kernel<true> : qz::thomas_lanes_kernel<false>,
                            dim3((batch + 3) / 4), dim3(64), 0, st, a, b, c, d, x, work, M, batch, sys_stride, elem_stride);
         QZ_HIP(hipGetLastError());
         return QZ_OK;
     }
     const int tb = 64;
-    hipLaunchKernelGGL(qz::thomas_batched_kernel, dim3((batch + tb - 1) / tb), dim3(tb), 0, st, a, b, c, d, x, work, M,
-                       batch, sys_stride, elem_stride);
+    hipLaunchKernelGGL(M <= kThomasTinyRows ? qz::thomas_batched_kernel<2> : qz::thomas_batched_kernel<8>,
+                       dim3((batch + tb - 1) / tb), dim3(tb), 0, st, a, b, c, d, x, work, M, batch, sys_stride, elem_stride);
     QZ_HIP(hipGetLastError());
     return QZ_OK;
 }
