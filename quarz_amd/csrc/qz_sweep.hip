@@ -15,7 +15,7 @@ __global__ __launch_bounds__(kBS) void sweep_kernel(const qz_sweep_args* __restr
 // LDS bytes of the runs that the one-workgroup sweep takes: N cells, PT particles per thread, L live particles.  The
 // sort's arrays are counted beside the region they share with the lists: that room (its counters alone take 16 N bytes)
 // holds the lists' shifts (8 (N + 1) bytes).
-long sweep_lds_needed(bool m1, int N, int pt, int L) {
+constexpr long lds_needed(bool m1, int N, int pt, int L) {
     const LdsPlan plan(N, pt);
     const long Mp = plan.Mp;
     const long nmax = m1 ? Lay<true>::NMAX : Lay<false>::NMAX;
@@ -25,6 +25,32 @@ long sweep_lds_needed(bool m1, int N, int pt, int L) {
     need = std::max(need, 2L * L);                // one deposit contribution list
     return plan.region + plan.sort + need * 8;
 }
+long sweep_lds_needed(bool m1, int N, int pt, int L) { return lds_needed(m1, N, pt, L); }
+
+// Room for `lists` components' lists (2 L + M doubles each) in every run of N cells and pt particles per thread that
+// lds_needed accepts: with as many live particles as it accepts.
+constexpr bool lists_fit(bool m1, int N, int pt, int lists) {
+    if (lds_needed(m1, N, pt, 0) > kLdsBytes) return true;
+    long lo = 0, hi = kBS * pt;   // the largest count accepted
+    while (lo < hi) {
+        const long mid = (lo + hi + 1) / 2;
+        if (lds_needed(m1, N, pt, static_cast<int>(mid)) <= kLdsBytes) lo = mid;
+        else hi = mid - 1;
+    }
+    return lists * (2 * lo + N + 1) <= (kLdsBytes - LdsPlan(N, pt).region) / 8;
+}
+// what the deposit's passes assume (qz_sweep_single.hpp): one list, and two in m = 1 and up to 4 particles per thread
+template <bool m1, int pt> constexpr bool deposit_lists_fit() {
+    for (int N = 2; lds_needed(m1, N, pt, 0) <= kLdsBytes; ++N)
+        if (!lists_fit(m1, N, pt, m1 || pt <= 4 ? 2 : 1)) return false;
+    return true;
+}
+static_assert(deposit_lists_fit<false, 2>());
+static_assert(deposit_lists_fit<false, 4>());
+static_assert(deposit_lists_fit<false, 8>());
+static_assert(deposit_lists_fit<true, 2>());
+static_assert(deposit_lists_fit<true, 4>());
+static_assert(deposit_lists_fit<true, 8>());
 
 }  // namespace qz
 

@@ -37,7 +37,8 @@ constexpr int kMiscBytes = 512;    // counters, bw0 of the chi factors, deposit 
 // lie at the start of the region: nothing else is in it while the particles are sorted.
 struct LdsPlan {
     int Mp, cs, misc, region, wcnt, sidx, sort;
-    __host__ __device__ LdsPlan(int N, int pt) {
+    __host__ __device__ constexpr LdsPlan(int N, int pt)
+        : Mp(0), cs(0), misc(0), region(0), wcnt(0), sidx(0), sort(0) {
         const int M = N + 1;
         Mp = (M + 1) & ~1;
         cs = 3 * Mp * 8;
@@ -502,8 +503,8 @@ __device__ __forceinline__ void sweep_run(const qz_sweep_args& A) {
                 gcur += n;
                 if (gcur >= G) reduce();
             };
-            // up to 2048 particles on a grid that fits, and in m = 1, two components always have room (G >= 2); a pass of
-            // four is taken where they have
+            // up to 2048 particles on a grid that fits, and in m = 1, two components always have room (G >= 2: asserted
+            // beside sweep_lds_needed for every run that it accepts); a pass of four is taken where they have
             if constexpr (!M1 && PT > 4) {
                 comp_pass(IC<W_CHI0>{});
                 comp_pass(IC<W_RHOT0>{});
