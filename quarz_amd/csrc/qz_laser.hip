@@ -11,8 +11,9 @@
 //     all nodes in LDS, one wave runs the right-hand side's Thomas recurrence and the back substitution (serial
 //     chains, as in the reference), and the workgroup forms the carry and a^(n+1).  The pivots and c' of the
 //     recurrence depend only on the slice's susceptibility, so the factor kernel forms them beforehand for all
-//     slices at once, one thread per slice, and the march's serial chain holds one complex division per node
-//     instead of two.  The carry stays in registers and the right-hand sides in LDS.
+//     slices at once, one thread per slice, and the march's serial chain holds one complex quotient per node
+//     instead of two: a product with a reciprocal, corrected, checked against the division, and divided where that
+//     differs (march_box).  The carry stays in registers and the right-hand sides in LDS.
 //
 // The arithmetic of each node follows the reference's expressions in the same order (no contraction), so the
 // result equals the serial CPU restatement bit for bit.  Scope: laser.l = 0 (no vortex), no ionization losses,
@@ -167,10 +168,13 @@ struct MarchLds {
 // passed through 64 nodes, which cost one set of LDS accesses (an LDS read costs the wave 9 to 14 cycles, a write 13 to
 // 27; one pair walking the nodes through LDS took 186 cycles per node).  A quotient n / |m|^2 in the chain is n y corrected once by its exact
 // residual, y = 1 / |m|^2 formed beforehand: three dependent operations against about twelve of a division.  The
-// correction gives the correctly rounded quotient but for operands at the ends of the exponent range, so while the
-// back substitution runs the other waves divide every node's numerator again with the IEEE division and compare the
-// bits; a slice with any difference has its chain run again with that division.  The next slice's rows and envelope
-// are loaded into registers while the chain runs, and the carry stays in its owner's registers.
+// correction gives the correctly rounded quotient but for operands at the ends of the exponent range, so every node's
+// numerator is divided again with the IEEE division and the bits compared: waves 1 to 7 do so while wave 0 runs the back
+// substitution, wave 0 for its own nodes after it.  A slice with any difference has its chain run again with that
+// division.  The next slice's rows and envelope are loaded beside the chain, and the carry stays in its owner's registers.
+// The three forms are one kernel, which takes all 256 registers and spills beside them (alone, NPT = 1 takes 230 and
+// spills none, 2 and 4 spill 40 and about 290); a compute unit so holds one march: 256 boxes of 513 nodes x 101 slices
+// 3.4 ms, 512 boxes 6.8 and 768 10.3, where the form of 66 registers, three to a unit, took 16.8, 21.6 and 25.4.
 // Measured on 401 slices x 321 nodes (bdf2): 6.8 ms a step, 41e3 cycles per slice, where one lane dividing in the
 // chain took 30.8 ms.
 // Every barrier is reached by all threads in every slice.

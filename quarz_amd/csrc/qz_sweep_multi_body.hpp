@@ -319,7 +319,8 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
     }
 
     int cj[PT], lrank[PT], cpos[PT];   // cell; rank; positions in this workgroup's own lists, left | right << 16
-    constexpr int kRows = PT <= 4 ? kChainR : 4;   // rows per lane of the chains: their registers beside the particles'
+    // rows per lane of the chains, as the one-workgroup kernel (here 8 rows beside 8 particles take no longer)
+    constexpr int kRows = PT <= 4 ? kChainR : 4;
     constexpr bool kMom = PT <= 2;                 // momenta, Delta and weight in registers for the slice
     constexpr int PM = kMom ? PT : 1, PB = PT <= 4 ? PT : 2;
     Real cpx[PM], cpy[PM], cdl[PM], cw[PM];
