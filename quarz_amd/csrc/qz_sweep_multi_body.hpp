@@ -545,8 +545,8 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
             // a wave sums the lists of eight nodes: eight lanes read 64 bytes of an entry side by side, a lane the same double
             // of each such part, and the sums of eight nodes are stored side by side.  Bound by the trips to memory: 29 us
             // a slice (m = 1, 1025 nodes, 64 entries a node, 8 workgroups), 42 us with the sources read after the sums,
-            // 9 and 18 us with 513 nodes and 16 entries.  11 entries in flight beside eight particles per thread: 12
-            // spill.
+            // 9 and 18 us with 513 nodes and 16 entries.  11 entries in flight beside eight particles per thread, where
+            // two registers spill (four with 12, 34 with 16).
             constexpr int P = SL::ENTRY / 8;
             for (int tile = grp * mNW + w; tile < (M + 7) / 8; tile += G * mNW) {
                 const int n = 8 * tile + (lane >> 3);
