@@ -53,10 +53,12 @@ constexpr unsigned long long kBarrierTicks = 200000000ull;   // 2 s of the 100 M
 // and stay in its L2, so a cache line lies between them and what the workgroups share, and after them.
 constexpr int kLineDoubles = 16;
 constexpr int kEntrySlots = 24;   // doubles of a list entry in m = 1 (8 in m = 0)
+// bw0 of the chi factors: lines away from the counters, which atomics change in place, and from the counts
+constexpr int kBw0 = 2 * kLineDoubles;
 struct MwsLayout {
     size_t misc = 0, cnt, lists, bpalt, gath, total;
     __host__ __device__ MwsLayout(int M, int N, int np, int G, bool m1) {
-        cnt = 64;   // words 0 barrier, 1 exit count, 2 error; doubles [8..12) bw0
+        cnt = 64;   // words 0 barrier, 1 exit count, 2 error; doubles [kBw0, kBw0 + 4) bw0
         lists = cnt + (static_cast<size_t>(G) * (N + 1) + 1) / 2 + 1;     // G x N ints
         lists = (lists + kLineDoubles - 1) / kLineDoubles * kLineDoubles;
         bpalt = lists + static_cast<size_t>(kEntrySlots) * 2 * (np > 1 ? np : 1);
@@ -268,7 +270,7 @@ __device__ __forceinline__ void sweep_multi_run(const qz_sweep_args* __restrict_
     Real* mws = A.mws;
     unsigned int* bar = reinterpret_cast<unsigned int*>(mws);
     unsigned int* err = bar + 2;
-    const Real* g_bw0 = mws + 8;
+    const Real* g_bw0 = mws + kBw0;
     const int* g_cnt = reinterpret_cast<const int*>(mws + mw.cnt);
     const Real* g_list = mws + mw.lists;
     const __amdgpu_buffer_rsrc_t list_buf = shared_buffer(g_list, mw.bpalt - mw.lists);
